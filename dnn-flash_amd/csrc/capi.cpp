@@ -296,9 +296,10 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
         r.tile_list = false;
         r.lds_list = false;
         r.paired = false;
-        r.block_m = 1;
-        r.block_n = 64;
-        r.threads = 256;
+        const bool blocks = ofh::row_blocks_take((int)p->head_dim, (int)p->value_dim);
+        r.block_m = blocks ? ofh::kRowBlock : 1;
+        r.block_n = blocks ? ofh::kRowBlock : 64;
+        r.threads = blocks ? ofh::kRowBlockThreads : 256;
         r.num_q_tiles = 0;
         r.num_k_tiles = 0;
         r.key_splits = 1;
@@ -932,10 +933,12 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
             name = pair_name.c_str();
         }
     } else {
-        info->block_m = 1;
-        info->block_n = 64;
-        info->threads = 256;
-        info->workgroups = ((int64_t)p->batch * p->heads * p->query_tokens + 3) / 4;
+        info->block_m = r.block_m;
+        info->block_n = r.block_n;
+        info->threads = r.threads;
+        info->workgroups = r.block_m == 1
+                               ? ((int64_t)p->batch * p->heads * p->query_tokens + 3) / 4
+                               : (int64_t)p->batch * p->heads * (((int64_t)p->query_tokens + r.block_m - 1) / r.block_m);
         info->key_splits = 1;
         name = "rowwise_fwd_kernel";
     }

@@ -181,6 +181,12 @@ struct QkScoreArgs {
 // Launchers; each returns the hipError_t of the launch.
 hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipStream_t s);
 hipError_t launch_rowwise(const FwdArgs& a, int dtype, hipStream_t s);
+// Exact two-pass calls run 32-row blocks of eight wavefronts on the matrix
+// cores up to these head dims (Q, and a K or V block per wavefront, in LDS),
+// wider heads a wavefront per row.
+inline bool row_blocks_take(int D, int Dv) { return D <= 256 && Dv <= 256; }
+constexpr int kRowBlock = 32;  // query rows per workgroup, keys per wavefront tile
+constexpr int kRowBlockThreads = 512;
 hipError_t launch_tile_lists(const TileListArgs& a, hipStream_t s);
 // Merge of the key-split partial rows into O in a second launch (num_splits > 1,
 // split_counters null); dtype is the input type.

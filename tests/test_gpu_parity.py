@@ -284,6 +284,44 @@ def test_rowwise_kernel_any_shape(ofh, dt):
     check(out, oracle_full(host, causal=True), dt, f"{dt} rowwise forced")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("D,Dv", [(1, 1), (63, 65), (64, 64), (75, 128), (129, 50), (256, 256), (257, 40), (40, 257)])
+def test_rowwise_row_blocks(ofh, dt, D, Dv):
+    """The 32-row blocks of the rowwise kernel at the edges of their 64-column
+    blocks, 32-row blocks and 32-key tiles (and the wide kernel past 256), in
+    [B,T,H,D] storage of no alignment, with a block mask that leaves some rows
+    empty; then with infinities and NaN in V, which reach the rows that give
+    their key a non-zero probability and no other. The error bound is the sums'
+    (n = D or N terms of 2^-24 each stay under the fp32 bar at these sizes)."""
+    for M, N, causal in [(1, 1, False), (33, 31, True), (64, 97, False), (70, 300, True)]:
+        dev, host = make_inputs(dt, 2, 2, M, N, D, Dv, seed=M + D)
+        dev = tuple(t.transpose(1, 2).contiguous().transpose(1, 2) for t in dev)
+        check(run(ofh, dev, dt=dt, causal=causal, algorithm=ofh.ALGO_ROWWISE), oracle_full(host, causal=causal),
+              dt, f"{dt} row blocks M{M} N{N} D{D} Dv{Dv}")
+    mask = (np.arange(5 * 7).reshape(5, 7) % 3 == 0).astype(np.uint8)
+    mask[2] = 0
+    out = run(ofh, dev, dt=dt, causal=True, mask=mask, mbs=(16, 40), algorithm=ofh.ALGO_ROWWISE)
+    ref = oracle_full(host, causal=True, mask=mask, mbs=(16, 40))
+    check(out, ref, dt, f"{dt} row blocks, block mask D{D} Dv{Dv}")
+    assert np.all(out[:, :, 32:48] == 0)
+    # the keys that no query row sees (causal, N > M) may hold anything
+    dev[2][:, :, 70:] = float("nan")
+    again = run(ofh, dev, dt=dt, causal=True, mask=mask, mbs=(16, 40), algorithm=ofh.ALGO_ROWWISE)
+    assert np.array_equal(out, again)
+    dev[2][0, 0, 20, 0] = float("inf")
+    dev[2][0, 1, 21, Dv - 1] = float("-inf")
+    dev[2][1, 0, 22, 0] = float("nan")
+    out = run(ofh, dev, dt=dt, causal=True, algorithm=ofh.ALGO_ROWWISE)
+    want = oracle_full(host, causal=True)
+    want[0, 0, 20:, 0] = np.inf
+    want[0, 1, 21:, Dv - 1] = -np.inf
+    want[1, 0, 22:, 0] = np.nan
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isfinite(out), finite)
+    assert np.array_equal(out[np.isinf(want)], want[np.isinf(want)])
+    assert_bars(norm_error(out[finite], want[finite])[0], dt, "finite rows beside non-finite V")
+
+
 def test_strided_layouts(ofh):
     B, H, M, N, D = 2, 4, 150, 170, 128
     dev, host = make_inputs("bf16", B, H, M, N, D, seed=13)
