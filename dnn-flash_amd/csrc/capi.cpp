@@ -49,6 +49,7 @@ struct Resolved {
     int key_splits;      // workgroups per query tile, each over a range of K/V tiles
     int split_tiles;     // K/V tile steps per split
     bool pair_split;     // causal: query tile pairs, each tile split in key_splits ranges of its own length
+    bool decode;         // a few query rows: flash_fwd_decode_kernel, one workgroup per head and key split
     int kdim;            // head dim of the MFMA kernel: max(D, Dv) rounded up to a multiple of 32
 };
 
@@ -143,6 +144,7 @@ int validate(const ofh_attention_params* p, bool check_ptrs, const void* q, cons
 // plain-scale block-mask kernels up to D = 64), the fp32 kernels two up to
 // D = 64.
 int workgroups_per_cu(const ofh_attention_params* p, const Resolved& r) {
+    if (r.decode) return 1;
     if (p->dtype == OFH_DTYPE_F32) return r.kdim <= 64 ? 2 : 1;
     if (r.threads >= 512) return 1;
     if (r.tile_list && !r.general_mod && r.kdim <= 64) return 3;
@@ -165,7 +167,7 @@ void choose_key_splits(const ofh_attention_params* p, Resolved& r) {
     r.pair_split = false;
     if (p->dtype == OFH_DTYPE_F32 && (r.paired || r.block_m == ofh::kRowsF32Narrow)) return;
     if (p->max_key_splits == 1) return;
-    const bool rows32 = p->dtype == OFH_DTYPE_F32 && r.block_m == ofh::kRowsF32;
+    const bool rows32 = !r.decode && p->dtype == OFH_DTYPE_F32 && r.block_m == ofh::kRowsF32;
     const int64_t slots = kComputeUnits * workgroups_per_cu(p, r);
     const int kMaxSplits = p->max_key_splits > 1 ? std::min(p->max_key_splits, 64) : 64;
     const int64_t bh = (int64_t)p->batch * p->heads;
@@ -205,9 +207,12 @@ void choose_key_splits(const ofh_attention_params* p, Resolved& r) {
         steps[(size_t)qt] = (int)((kend + r.block_n - 1) / r.block_n);
         max_steps = std::max(max_steps, steps[(size_t)qt]);
     }
+    // A decode call that one workgroup per head ends in two steps: the merge
+    // costs more (fp32 B1 H8 M1 N500 D64 5.4 us against 6.5 in two splits).
+    if (r.decode && max_steps <= 2) return;
     // at least 64 keys per split (128/256-row kernels), or a tile per
     // wavefront (32-row fp32 blocks)
-    const int min_steps = rows32 ? 4 : std::max(1, 64 / r.block_n);
+    const int min_steps = r.decode ? 1 : rows32 ? 4 : std::max(1, 64 / r.block_n);
     const int most = std::min(kMaxSplits, std::max(1, max_steps / min_steps));
     auto per_of = [&](int n) { return (max_steps + n - 1) / n; };
     auto active = [&](int n) {
@@ -246,7 +251,8 @@ void no_key_split(const ofh_attention_params* p, Resolved& r) {
     r.key_splits = 1;
     r.split_tiles = 1 << 30;
     r.pair_split = false;
-    // 32- and 16-row blocks: no pairing, no list
+    // decode kernel, 32- and 16-row blocks: no pairing, no list
+    if (r.decode) return;
     if (p->dtype == OFH_DTYPE_F32 && (r.block_m == ofh::kRowsF32 || r.block_m == ofh::kRowsF32Narrow)) return;
     const ofh::MfmaTiles t = ofh::flash_mfma_tiles(p->dtype, r.kdim, r.general_mod, r.tile_list, p->causal != 0,
                                                    (int64_t)p->batch * p->heads, p->query_tokens);
@@ -263,6 +269,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     contiguous_strides(r.vs, p->v_strides, p->heads, p->key_tokens, p->value_dim);
     contiguous_strides(r.os, p->o_strides, p->heads, p->query_tokens, p->value_dim);
     r.general_mod = p->bias_kind != OFH_BIAS_NONE || p->softcap > 0.0f;
+    r.decode = false;
 
     // The MFMA kernels read and write 16-byte row chunks.
     const size_t es = elem_size(p->dtype), oes = elem_size(p->out_dtype);
@@ -318,9 +325,22 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     r.num_q_tiles = (int)((p->query_tokens + r.block_m - 1) / r.block_m);
     r.num_k_tiles = (int)((p->key_tokens + r.block_n - 1) / r.block_n);
     r.tile_list = p->mask_allowed != nullptr;
+    // A few query rows (decoding), plain scale and no mask: the vector kernel
+    // that streams K and V through registers. Planned as one 32-row query
+    // block per head. (2^30: its key positions are 32-bit sums.)
+    r.decode = p->algorithm == OFH_ALGO_AUTO && !r.tile_list && !r.general_mod && !p->causal &&
+               (int64_t)p->query_tokens <= ofh::decode_max_rows(p->dtype, (int)p->head_dim, (int)p->value_dim) && p->key_tokens >= (size_t)ofh::kDecodeMinKeys && p->key_tokens <= (size_t)1 << 30;
+    if (r.decode) {
+        r.block_m = 32;
+        r.block_n = ofh::decode_step_keys(p->dtype, (int)p->head_dim, (int)p->value_dim);
+        r.threads = ofh::kDecodeThreads;
+        r.paired = false;
+        r.num_q_tiles = 1;
+        r.num_k_tiles = (int)((p->key_tokens + r.block_n - 1) / r.block_n);
+    }
     // fp32 with few query tiles (latency-bound): 32-row query blocks whose
     // four wavefronts share the keys, 32-key tiles (built up to D = 128)
-    if (p->dtype == OFH_DTYPE_F32 && !r.tile_list && r.kdim <= 128 &&
+    if (!r.decode && p->dtype == OFH_DTYPE_F32 && !r.tile_list && r.kdim <= 128 &&
         (int64_t)p->batch * p->heads * r.num_q_tiles < ofh::kRows32Below) {
         r.block_m = ofh::kRowsF32;
         r.block_n = 32;
@@ -685,7 +705,8 @@ int fwd_impl(const ofh_attention_params* p, const void* q, const void* k, const 
         if (merge_in_launch(p, r))
             if (int rc = split_counters_for(stream, noalloc, &a.split_counters)) return rc;
     }
-    OFH_HIP_CHECK(ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
+    OFH_HIP_CHECK(r.decode ? ofh::launch_decode(a, p->dtype, stream)
+                           : ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
     if (r.key_splits > 1 && a.split_counters == nullptr)
         OFH_HIP_CHECK(ofh::launch_combine_splits(a, p->dtype, stream));
     if (shared != nullptr) {
@@ -871,6 +892,18 @@ int ofh_attention_fwd_host(const ofh_attention_params* p, const float* q, const 
 }
 
 namespace {
+const char* decode_kernel_name(int dtype, int D, int Dv) {
+    static const std::vector<std::string> names = [] {
+        std::vector<std::string> v;
+        for (const char* t : {"f32", "bf16", "f16"})
+            for (int lanes = 8; lanes <= 64; lanes *= 2)
+                v.push_back(std::string("flash_fwd_decode_kernel<") + t + "," +
+                            std::to_string(lanes * (t[0] == 'f' && t[1] == '3' ? 4 : 8)) + ">");
+        return v;
+    }();
+    const int lanes = ofh::decode_row_lanes(dtype, D, Dv);
+    return names[(size_t)dtype * 4 + (lanes == 8 ? 0 : lanes == 16 ? 1 : lanes == 32 ? 2 : 3)].c_str();
+}
 const char* rows32_kernel_name(int D, bool general, bool narrow) {
     static const std::vector<std::string> names = [] {
         std::vector<std::string> v;
@@ -903,7 +936,8 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
                            r.key_splits;
         info->key_splits = r.key_splits;
         info->merge_in_launch = merge_in_launch(p, r) ? 1 : 0;
-        name = (p->dtype == OFH_DTYPE_F32 && (r.block_m == ofh::kRowsF32 || r.block_m == ofh::kRowsF32Narrow))
+        name = r.decode ? decode_kernel_name(p->dtype, (int)p->head_dim, (int)p->value_dim)
+               : (p->dtype == OFH_DTYPE_F32 && (r.block_m == ofh::kRowsF32 || r.block_m == ofh::kRowsF32Narrow))
                    ? rows32_kernel_name(r.kdim, r.general_mod, r.block_m == ofh::kRowsF32Narrow)
                    : ofh::flash_mfma_kernel_name(p->dtype, r.kdim, r.general_mod, r.tile_list, r.threads);
         // 16-bit causal pairs with a key split run the same tiling in a kernel of their own

@@ -180,6 +180,35 @@ struct QkScoreArgs {
 
 // Launchers; each returns the hipError_t of the launch.
 hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipStream_t s);
+// Calls with a few query rows (decode_fwd.hip): plain scale, no mask.
+hipError_t launch_decode(const FwdArgs& a, int dtype, hipStream_t s);
+constexpr int kDecodeThreads = 512;
+// Query rows the decode kernel takes. A 16-bit row costs unpacking V and the
+// products on the vector units: bf16 B8 H32 N4096 D128 89.9 us at one row
+// against 92.0 on the matrix cores (where the error against 64 bits is larger,
+// probabilities being rounded to bf16), 96.9 against 92.4 at four and 136
+// against 93 at eight. fp32 B16 H16 N4096 D64 stays at the memory's rate up to
+// eight (111 us; 90 at one row, against 300 on the matrix cores).
+// 16-bit heads wider than 128 keep the matrix-core kernels (not measured here).
+inline int decode_max_rows(int dtype, int D, int Dv) {
+    return dtype == DT_F32 ? 8 : D <= 128 && Dv <= 128 ? 2 : 0;
+}
+// Fewer keys are no stream: such calls take a launch's latency on any kernel.
+constexpr int kDecodeMinKeys = 64;
+// Lanes that hold a K or V row of the decode kernel, 16 bytes each.
+inline int decode_row_lanes(int dtype, int D, int Dv) {
+    const int chunks = (D > Dv ? D : Dv) / (dtype == DT_F32 ? 4 : 8);
+    return chunks <= 8 ? 8 : chunks <= 16 ? 16 : chunks <= 32 ? 32 : 64;
+}
+// Load instructions (64 / lanes rows each) per wavefront and group of keys. 4,
+// 6 and 8 measured within 4 % of each other up to two query rows (bf16 B8 H32
+// M1 N4096 D128 89.9, 90.8, 93.4 us; fp32 B1 H16 M1 N4096 D64 10.8, 10.2,
+// 10.8); with more rows, 8 spill.
+constexpr int kDecodeLoads = 4;
+// Keys per step of a workgroup: a group of every wavefront.
+inline int decode_step_keys(int dtype, int D, int Dv) {
+    return kDecodeThreads / 64 * kDecodeLoads * (64 / decode_row_lanes(dtype, D, Dv));
+}
 hipError_t launch_rowwise(const FwdArgs& a, int dtype, hipStream_t s);
 // Exact two-pass calls run 32-row blocks of eight wavefronts on the matrix
 // cores up to these head dims (Q, and a K or V block per wavefront, in LDS),

@@ -219,7 +219,7 @@ __global__ __launch_bounds__(64 * NW) void rowwise_fwd_kernel(FwdArgs a, int num
     const float* bias_row =
         a.bias_kind == BIAS_DENSE ? a.bias + b * a.bias_sb + h * a.bias_sh + (int64_t)qi * a.bias_sm : nullptr;
     const int kend = a.causal ? (int)min((int64_t)a.N, (int64_t)q0 + kRowBlock) : a.N;
-    const int ntiles = (kend + kRowBlock - 1) / kRowBlock;
+    const int ntiles = (int)(((int64_t)kend + kRowBlock - 1) / kRowBlock);
 
     // Bit e: key rw_key(e, g) of tile t is valid for this lane's row.
     auto valid_keys = [&](int t) {

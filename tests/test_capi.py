@@ -268,6 +268,20 @@ def test_kernel_choice(ofh):
         (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=160), "flash_fwd_mfma32_kernel<160,plain>"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=264), "rowwise_fwd_kernel"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, algorithm=F.ALGO_ROWWISE), "rowwise_fwd_kernel"),
+        # a few query rows (8 fp32, 2 16-bit), plain scale, no mask: the decode kernel
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 8, 200)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 9, 200)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=80, shape=(2, 3, 2, 200)), "flash_fwd_decode_kernel<bf16,128>"),
+        (dict(dtype=F.DTYPE_F16, head_dim=64, value_dim=128, shape=(2, 3, 1, 200)), "flash_fwd_decode_kernel<f16,128>"),
+        (dict(dtype=F.DTYPE_F16, head_dim=136, shape=(2, 3, 1, 200)), "flash_fwd_lockstep_kernel<f16,160,plain,8w,2x64keys>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=256, shape=(2, 3, 5, 200)), "flash_fwd_decode_kernel<f32,256>"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=128, shape=(2, 3, 3, 200)), "flash_fwd_lockstep_kernel<bf16,128,plain,8w,2x64keys>"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=128, shape=(2, 3, 1, 200), causal=True),
+         "flash_fwd_lockstep_kernel<bf16,128,plain,8w,2x64keys>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 1, 63)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=128, shape=(2, 3, 1, 200), softcap=5.0), "flash_fwd_lockstep_kernel<bf16,128,mod,8w>"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=128, shape=(2, 3, 1, 200), algorithm=F.ALGO_FLASH_MFMA),
+         "flash_fwd_lockstep_kernel<bf16,128,plain,8w,2x64keys>"),
     ]
     for kw, name in cases:
         D = kw.pop("head_dim")
