@@ -49,6 +49,7 @@ struct Resolved {
     int key_splits;      // workgroups per query tile, each over a range of K/V tiles
     int split_tiles;     // K/V tile steps per split
     bool pair_split;     // causal: query tile pairs, each tile split in key_splits ranges of its own length
+    int groups;          // > 0: wavefront groups split the keys inside a workgroup (flash_fwd_keygroups_kernel)
     bool decode;         // a few query rows: flash_fwd_decode_kernel, one workgroup per head and key split
     int kdim;            // head dim of the MFMA kernel: max(D, Dv) rounded up to a multiple of 32
 };
@@ -262,6 +263,70 @@ void no_key_split(const ofh_attention_params* p, Resolved& r) {
     set_lds_list(p, r);
 }
 
+// 16-bit plain-scale calls that the planner would split over workgroups (few
+// query tiles, so without a split CUs stay idle) run wavefront groups instead
+// where those are faster: no partial rows in memory and no merge launch, but
+// each staged K/V tile serves 1/groups of the query rows.
+//
+// The estimate of a plan is its rounds of workgroups over the CUs (prologue,
+// fold and store of each) and the staged tiles of the longest chain of one CU;
+// the constants are a fit to 290 shapes per head dim (H 1-128, N 100-16000,
+// causal and not; 80 % within 9 %). Measured bounds (us, split against the
+// better group count): bf16 D128 causal H32 N1000 43 / 24, H8 N2048 42 / 28, H4
+// N2500 42 / 32, H8 N4096 55 / 58, non-causal H8 N1000 31 / 18, H8 N4096 80 /
+// 74, H16 M500 N4000 36 / 54: from about 38 us (30 at kernel dim 96, 26 up to
+// 64) the chain outweighs what the merge costs. Causal pairs split in ranges
+// of their own lose less, hence their lower line (H128 N512 55 / 33, H32 N2048
+// 68 / 70). Few rows (one 128-row tile) leave groups without their gain (H64
+// M64 N1000 16 / 18), and grids of less than 32 128-row tiles keep the split,
+// on whose workspace and launch description their callers may rely.
+void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
+    if (p->dtype == OFH_DTYPE_F32 || p->max_key_splits != 0 || r.key_splits <= 1 || r.decode || r.general_mod ||
+        r.tile_list || r.kdim > 128 || p->query_tokens <= 128)
+        return;
+    const int64_t bh = (int64_t)p->batch * p->heads, M = (int64_t)p->query_tokens, N = (int64_t)p->key_tokens;
+    if (bh * ((M + 127) / 128) < 32) return;
+    struct Fit {
+        float base, round, tile;  // us
+    };
+    const Fit fits[3][2] = {{{-1.2f, 6.8f, 1.27f}, {0.9f, 4.5f, 1.50f}},   // kernel dim 32, 64: 2, 4 groups
+                            {{-0.1f, 5.5f, 1.70f}, {-1.5f, 7.4f, 1.20f}},  // 96
+                            {{-5.5f, 12.6f, 1.83f}, {-0.5f, 8.0f, 1.28f}}};  // 128
+    const int dim = r.kdim <= 64 ? 0 : r.kdim <= 96 ? 1 : 2;
+    int best = 0;
+    float best_us = 0.0f;
+    for (int groups = 2; groups <= 4; groups += 2) {
+        const int64_t rows = 8 * ofh::kQueriesPerWave / groups, keys = ofh::key_group_keys(r.kdim, groups);
+        const int64_t tiles = (M + rows - 1) / rows, wgs = bh * tiles;
+        const int64_t rounds = (wgs + kComputeUnits - 1) / kComputeUnits;
+        int64_t longest = 0, total = 0;
+        for (int64_t t = 0; t < tiles; ++t) {
+            const int64_t kend = p->causal ? std::min(N, (t + 1) * rows) : N;
+            const int64_t steps = (kend + keys - 1) / keys;
+            longest = std::max(longest, steps);
+            total += steps;
+        }
+        // causal workgroups differ in length and are handed out longest first
+        const int64_t chain = p->causal ? std::max(longest, (total * bh + kComputeUnits - 1) / kComputeUnits)
+                                        : rounds * longest;
+        const Fit& f = fits[dim][groups / 2 - 1];
+        const float us = f.base + f.round * (float)rounds + f.tile * (float)chain;
+        if (best == 0 || us < best_us) {
+            best = groups;
+            best_us = us;
+        }
+    }
+    const float line[3] = {26.0f, 30.0f, 38.0f};
+    if (best_us > line[dim] * (r.pair_split ? 0.8f : 1.0f)) return;
+    no_key_split(p, r);
+    r.groups = best;
+    r.paired = false;
+    r.block_m = 8 * ofh::kQueriesPerWave / best;
+    r.block_n = ofh::key_group_keys(r.kdim, best);
+    r.num_q_tiles = (int)((M + r.block_m - 1) / r.block_m);
+    r.num_k_tiles = (int)((N + r.block_n - 1) / r.block_n);
+}
+
 int resolve(const ofh_attention_params* p, const void* q, const void* k, const void* v,
             const void* out, Resolved& r) {
     contiguous_strides(r.qs, p->q_strides, p->heads, p->query_tokens, p->head_dim);
@@ -270,6 +335,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     contiguous_strides(r.os, p->o_strides, p->heads, p->query_tokens, p->value_dim);
     r.general_mod = p->bias_kind != OFH_BIAS_NONE || p->softcap > 0.0f;
     r.decode = false;
+    r.groups = 0;
 
     // The MFMA kernels read and write 16-byte row chunks.
     const size_t es = elem_size(p->dtype), oes = elem_size(p->out_dtype);
@@ -379,6 +445,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     if (r.tile_list && (r.block_m > ofh::kQueriesPerWave * ofh::kListSlices || r.num_k_tiles > (1 << 22)))
         return set_error(OFH_ERROR_UNSUPPORTED, "block-mask tile list entry cannot encode this tiling");
     choose_key_splits(p, r);
+    choose_key_groups(p, r);
     set_lds_list(p, r);
     return OFH_SUCCESS;
 }
@@ -705,8 +772,9 @@ int fwd_impl(const ofh_attention_params* p, const void* q, const void* k, const 
         if (merge_in_launch(p, r))
             if (int rc = split_counters_for(stream, noalloc, &a.split_counters)) return rc;
     }
-    OFH_HIP_CHECK(r.decode ? ofh::launch_decode(a, p->dtype, stream)
-                           : ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
+    OFH_HIP_CHECK(r.groups   ? ofh::launch_key_groups(a, p->dtype, r.groups, stream)
+                  : r.decode ? ofh::launch_decode(a, p->dtype, stream)
+                             : ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
     if (r.key_splits > 1 && a.split_counters == nullptr)
         OFH_HIP_CHECK(ofh::launch_combine_splits(a, p->dtype, stream));
     if (shared != nullptr) {
@@ -940,9 +1008,15 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
                : (p->dtype == OFH_DTYPE_F32 && (r.block_m == ofh::kRowsF32 || r.block_m == ofh::kRowsF32Narrow))
                    ? rows32_kernel_name(r.kdim, r.general_mod, r.block_m == ofh::kRowsF32Narrow)
                    : ofh::flash_mfma_kernel_name(p->dtype, r.kdim, r.general_mod, r.tile_list, r.threads);
-        // 16-bit causal pairs with a key split run the same tiling in a kernel of their own
         static thread_local std::string pair_name;
         const std::string lockstep = "flash_fwd_lockstep_kernel";
+        // wavefront groups that split the keys inside a workgroup
+        if (r.groups > 0) {
+            pair_name = std::string("flash_fwd_keygroups_kernel<") + (p->dtype == OFH_DTYPE_BF16 ? "bf16," : "f16,") +
+                        std::to_string(r.kdim) + ",plain," + std::to_string(r.groups) + "groups>";
+            name = pair_name.c_str();
+        }
+        // 16-bit causal pairs with a key split run the same tiling in a kernel of their own
         if (r.pair_split && p->dtype != OFH_DTYPE_F32 && std::string(name).compare(0, lockstep.size(), lockstep) == 0) {
             pair_name = "flash_fwd_pair_split_kernel" + std::string(name).substr(lockstep.size());
             name = pair_name.c_str();

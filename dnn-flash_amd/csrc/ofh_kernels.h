@@ -180,6 +180,12 @@ struct QkScoreArgs {
 
 // Launchers; each returns the hipError_t of the launch.
 hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipStream_t s);
+// 16-bit calls whose eight wavefronts split the keys of 256 / groups query rows
+// (flash_keygroups.hip), groups = 2 or 4; kernel head dims up to 128, plain
+// scale, no block mask, no key split over workgroups.
+hipError_t launch_key_groups(const FwdArgs& a, int dtype, int groups, hipStream_t s);
+// Keys of a staged tile: what one step of all groups covers.
+int key_group_keys(int kernel_dim, int groups);
 // Calls with a few query rows (decode_fwd.hip): plain scale, no mask.
 hipError_t launch_decode(const FwdArgs& a, int dtype, hipStream_t s);
 constexpr int kDecodeThreads = 512;

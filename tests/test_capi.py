@@ -377,6 +377,38 @@ def test_kernel_choice(ofh):
     _expect_error(F, p, F.OFH_ERROR_UNSUPPORTED, "token strides")
 
 
+def test_key_group_choice(ofh):
+    """Wavefront groups replace the key split over workgroups of 16-bit plain
+    calls with at least 32 query tiles of 128 rows and short chains; every
+    other call keeps its plan."""
+    F = ofh
+
+    def name(B, H, M, N, D, **kw):
+        return F.launch_info(F.make_params(B, H, M, N, D, dtype=F.DTYPE_BF16, **kw)).kernel_name.decode()
+
+    groups = "flash_fwd_keygroups_kernel<bf16,"
+    assert name(1, 32, 1000, 1000, 128, causal=True) == groups + "128,plain,2groups>"
+    assert name(1, 32, 512, 512, 128, causal=True) == groups + "128,plain,4groups>"
+    assert name(1, 8, 1000, 1000, 64) == groups + "64,plain,4groups>"
+    assert name(2, 8, 1000, 1000, 80) == groups + "96,plain,4groups>"
+    assert name(1, 128, 512, 512, 128, causal=True) == groups + "128,plain,2groups>"  # pairs that would split
+    p = F.make_params(1, 32, 1000, 1000, 128, dtype=F.DTYPE_BF16, causal=True)
+    info = F.launch_info(p)
+    assert info.block_m == 128 and info.block_n == 128 and info.threads == 512 and info.workgroups == 32 * 8
+    assert info.key_splits == 1 and F.workspace_bytes(p) == 0
+    for other in [name(1, 32, 1000, 1000, 128, causal=True, max_key_splits=1),
+                  name(1, 32, 1000, 1000, 128, causal=True, max_key_splits=2),
+                  name(1, 32, 1000, 1000, 128, causal=True, softcap=5.0),
+                  name(1, 32, 1000, 1000, 160, causal=True),
+                  name(1, 10, 300, 300, 128),         # 30 tiles of 128 rows
+                  name(1, 64, 128, 1000, 128),        # one tile of rows per head
+                  name(1, 8, 4096, 4096, 128, causal=True),
+                  name(1, 32, 2048, 2048, 128, causal=True),
+                  name(1, 32, 4096, 4096, 128, causal=True),
+                  F.launch_info(F.make_params(2, 16, 1000, 1000, 64)).kernel_name.decode()]:
+        assert "keygroups" not in other, other
+
+
 def test_useful_flops_match_workloads(ofh):
     import onednn_flash_configs as C
     F = ofh
