@@ -50,6 +50,7 @@ struct Resolved {
     int split_tiles;     // K/V tile steps per split
     bool pair_split;     // causal: query tile pairs, each tile split in key_splits ranges of its own length
     int groups;          // > 0: wavefront groups split the keys inside a workgroup (flash_fwd_keygroups_kernel)
+    bool staged_bias;    // 16-bit dense bias copied through LDS (flash_fwd_bias_kernel)
     bool decode;         // a few query rows: flash_fwd_decode_kernel, one workgroup per head and key split
     int kdim;            // head dim of the MFMA kernel: max(D, Dv) rounded up to a multiple of 32
 };
@@ -336,6 +337,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     r.general_mod = p->bias_kind != OFH_BIAS_NONE || p->softcap > 0.0f;
     r.decode = false;
     r.groups = 0;
+    r.staged_bias = false;
 
     // The MFMA kernels read and write 16-byte row chunks.
     const size_t es = elem_size(p->dtype), oes = elem_size(p->out_dtype);
@@ -391,6 +393,8 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     r.num_q_tiles = (int)((p->query_tokens + r.block_m - 1) / r.block_m);
     r.num_k_tiles = (int)((p->key_tokens + r.block_n - 1) / r.block_n);
     r.tile_list = p->mask_allowed != nullptr;
+    // (above 128 the K/V stages leave no room for the bias tiles in LDS)
+    r.staged_bias = p->dtype != OFH_DTYPE_F32 && p->bias_kind == OFH_BIAS_DENSE && !r.tile_list && r.kdim <= 128;
     // A few query rows (decoding), plain scale and no mask: the vector kernel
     // that streams K and V through registers. Planned as one 32-row query
     // block per head. (2^30: its key positions are 32-bit sums.)
@@ -772,7 +776,8 @@ int fwd_impl(const ofh_attention_params* p, const void* q, const void* k, const 
         if (merge_in_launch(p, r))
             if (int rc = split_counters_for(stream, noalloc, &a.split_counters)) return rc;
     }
-    OFH_HIP_CHECK(r.groups   ? ofh::launch_key_groups(a, p->dtype, r.groups, stream)
+    OFH_HIP_CHECK(r.staged_bias ? ofh::launch_bias(a, p->dtype, stream)
+                  : r.groups ? ofh::launch_key_groups(a, p->dtype, r.groups, stream)
                   : r.decode ? ofh::launch_decode(a, p->dtype, stream)
                              : ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
     if (r.key_splits > 1 && a.split_counters == nullptr)
@@ -1010,6 +1015,11 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
                    : ofh::flash_mfma_kernel_name(p->dtype, r.kdim, r.general_mod, r.tile_list, r.threads);
         static thread_local std::string pair_name;
         const std::string lockstep = "flash_fwd_lockstep_kernel";
+        if (r.staged_bias) {
+            pair_name = std::string("flash_fwd_bias_kernel<") + (p->dtype == OFH_DTYPE_BF16 ? "bf16," : "f16,") +
+                        std::to_string(r.kdim) + (r.pair_split ? ",pair split>" : r.paired ? ",paired>" : ">");
+            name = pair_name.c_str();
+        }
         // wavefront groups that split the keys inside a workgroup
         if (r.groups > 0) {
             pair_name = std::string("flash_fwd_keygroups_kernel<") + (p->dtype == OFH_DTYPE_BF16 ? "bf16," : "f16,") +

@@ -143,7 +143,9 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
 // Score modification of a 16-bit kernel instantiation: the plain scale, or
 // any mix of ALiBi / dense bias / soft-cap selected per call.
-enum ScoreMod { MOD_PLAIN = 0, MOD_GENERAL = 1 };
+// MOD_DENSE: a dense bias (with or without a soft-cap) whose tiles are copied
+// to LDS ahead of their use (flash_bias.hip).
+enum ScoreMod { MOD_PLAIN = 0, MOD_GENERAL = 1, MOD_DENSE = 2 };
 
 
 // One 16-byte global -> LDS copy per lane (lane L writes lds + 16 L; lds is
@@ -154,6 +156,19 @@ __device__ __forceinline__ void dma16(const void* g, unsigned lds) {
     unsigned save;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
                  : "=&s"(save) : "v"(g), "s"(lds) : "memory");
+}
+
+// The same from a wave-uniform base plus a per-lane byte offset, 16 or 4 bytes
+// per lane (lane L writes lds + 16 L or lds + 4 L).
+__device__ __forceinline__ void dma16s(const void* base, unsigned off, unsigned lds) {
+    unsigned save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(save) : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void dma4(const void* base, unsigned off, unsigned lds) {
+    unsigned save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(save) : "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
 // K and V tiles in LDS: row-major [key][d], unpadded (each global -> LDS
@@ -273,7 +288,8 @@ struct Wave32 {
     float m_run, l_run;
     float slope;
     float alibi_step[8];  // soft-capped ALiBi: 2^(slope c_b t), t = 0..7 (wave-uniform)
-    const float* bias_row;
+    const float* bias_row;  // this lane's row; MOD_DENSE: the head's first row
+    int bias_lds;           // MOD_DENSE: LDS offset of this wavefront's bias rows
     // LDS read lane offsets
     int k_lane_off, v_lane_off;
     // rows that are not a power of two wide: per-lane bases of the swizzled
@@ -344,6 +360,7 @@ struct Wave32 {
             if (a.bias_kind == BIAS_DENSE)
                 bias_row = a.bias + b * a.bias_sb + h * a.bias_sh + (int64_t)min(my_q, a.M - 1) * a.bias_sm;
         }
+        if (MOD == MOD_DENSE) bias_row = a.bias + b * a.bias_sb + h * a.bias_sh;
         // K: A-operand row kappa(r) of a 32-key block, chunk 2c+g. V (transposed
         // reads): input lane j of a 16-lane group reads key (j/4) of a 4-key
         // group at d-chunk cmap(j%4) of the group's 16 columns; cmap = {0,2,1,3}
@@ -446,6 +463,53 @@ struct Wave32 {
         }
     }
 
+    // MOD_DENSE: the bias of compute step e for this wavefront's 32 rows, copied
+    // global -> LDS (asynchronous) into 32 rows of BN floats of its own at
+    // bias_lds. 16-byte chunk c of row r sits at chunk c ^ (r & 15): a read
+    // takes one chunk of 16 rows, 256 bytes apart. Rows past M and keys past N
+    // repeat the last one (their scores are masked or never stored). VEC:
+    // 16-byte aligned rows and N a multiple of 4, eight copies of four rows;
+    // else 32 of one row, 4 bytes per lane.
+    static constexpr int BIAS_BYTES = 32 * BN * 4;  // per wavefront
+    template <bool VEC>
+    __device__ __forceinline__ void copy_bias(int e) {
+        static_assert(BN == 64, "a bias row is 16 chunks");
+        const int k0 = e * BN;
+        const unsigned lds0 = (unsigned)(uintptr_t)smem + bias_lds;
+        const float* base = bias_row + (int64_t)min(qw0, a.M - 1) * a.bias_sm + k0;  // uniform
+        // (the lane is hidden from the compiler so that the copies' offsets are
+        // formed here each time instead of kept in registers: at D = 128 those spill)
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
+        if (VEC && k0 + BN <= a.N && qw0 + kQueriesPerWave <= a.M) {
+            // copy u: rows 4u + lane / 16, chunk (lane % 16) ^ (lane / 16) ^ 4 (u % 4)
+            const unsigned roff = 4u * (unsigned)((lane >> 4) * (int)a.bias_sm);
+            const unsigned c0 = 16u * (unsigned)((lane & 15) ^ (lane >> 4));
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                dma16s(base, (c0 ^ (64u * (u & 3))) + roff, lds0 + 1024 * u);
+                base += 4 * a.bias_sm;
+            }
+        } else if constexpr (VEC) {
+            const int last_row = max(0, a.M - 1 - qw0), last = a.N - 4 - k0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int row = 4 * u + (lane >> 4);
+                const int key = min(4 * ((lane & 15) ^ (row & 15)), last);
+                dma16s(base, 4u * (unsigned)(min(row, last_row) * (int)a.bias_sm + key), lds0 + 1024 * u);
+            }
+        } else {
+            const unsigned off0 = 4u * (unsigned)lane, last = 4u * (unsigned)(a.N - 1 - k0);
+            int rows = a.M - qw0;  // likewise: 32 row conditions kept would spill scalar registers
+            asm volatile("" : "+s"(rows));
+#pragma unroll
+            for (int u = 0; u < 32; ++u) {
+                dma4(base, min(off0 ^ (16u * (u & 15)), last), lds0 + 256 * u);
+                base += u + 1 < rows ? a.bias_sm : 0;
+            }
+        }
+    }
+
     // S^T = K Q^T for the tile in LDS stage `stage_off`.
     __device__ __forceinline__ void qk(int stage_off, int sub = 0) {
         // Fragments are read kFragAhead MFMAs ahead of their use; the
@@ -512,7 +576,17 @@ struct Wave32 {
         const float sl = slope * c_b;
         const float base = sl * (float)(k0 + 8 * g - my_q);
         float bvals[BN / 2];
-        if (BIAS == BIAS_DENSE) {
+        if constexpr (MOD == MOD_DENSE) {
+            const lds_u8* br = (const lds_u8*)smem + bias_lds + (my_q - qw0) * BN * 4;
+            const int sw = (my_q - qw0) & 15;
+#pragma unroll
+            for (int q4 = 0; q4 < BN / 8; ++q4) {  // keys 16 (q4 >> 1) + 8 g + 4 (q4 & 1) .. + 3
+                const f32x4 v = __builtin_bit_cast(
+                    f32x4, *(const lds_u32x4*)(br + 16 * ((4 * (q4 >> 1) + 2 * g + (q4 & 1)) ^ sw)));
+#pragma unroll
+                for (int t = 0; t < 4; ++t) bvals[4 * q4 + t] = v[t];
+            }
+        } else if (BIAS == BIAS_DENSE) {
             const float* br = bias_row + k0 + 8 * g;
             if (k0 + BN <= a.N) {
 #pragma unroll
@@ -552,6 +626,8 @@ struct Wave32 {
                 float u;
                 if (BIAS == BIAS_ALIBI)
                     u = __builtin_fmaf(s[sb][e], c_s, __builtin_fmaf(sl, (float)tile_pos(sb, e), base));
+                else if (MOD == MOD_DENSE && !CAP)  // natural units: the softmax's exp2 argument applies log2e
+                    u = __builtin_fmaf(s[sb][e], a.scale, bvals[16 * sb + e]);
                 else if (BIAS == BIAS_DENSE)
                     u = __builtin_fmaf(s[sb][e], c_s, bvals[16 * sb + e] * c_b);
                 else
@@ -564,6 +640,11 @@ struct Wave32 {
     }
     __device__ __forceinline__ void general_scores(int k0) {
         const bool cap = a.softcap > 0.0f;
+        if constexpr (MOD == MOD_DENSE) {
+            if (cap) score_mod_tile<BIAS_DENSE, true>(k0);
+            else score_mod_tile<BIAS_DENSE, false>(k0);
+            return;
+        }
         if (a.bias_kind == BIAS_ALIBI) {
             if (cap) score_mod_tile<BIAS_ALIBI, true>(k0);
             else score_mod_tile<BIAS_ALIBI, false>(k0);
@@ -622,7 +703,15 @@ struct Wave32 {
         const int k0 = kt * BN;
         const bool need_mask = tile_crosses(kt) || (LIST && !list_full(e_ent, wave));
         float mx = kNegInf;
-        const bool raw = MOD == MOD_PLAIN && !need_mask;  // s still holds raw dot products
+        const bool capped = MOD != MOD_PLAIN && a.softcap > 0.0f;  // uniform
+        const bool natural = MOD == MOD_DENSE && !capped;          // s in natural units
+        if (natural) {
+            general_scores(k0);
+            if (need_mask) apply_mask(e_ent, k0);
+        }
+        // s still holds raw dot products (or natural scores): the log2 score is s * to_log2
+        const bool raw = (MOD == MOD_PLAIN && !need_mask) || natural;
+        const float to_log2 = MOD == MOD_DENSE ? kLog2e : a.scale_log2;
         // 128-key tiles (D <= 64, no list): p is taken against the running max
         // first, without the tile's max. A row sum of at most 2^kRescaleSlack
         // proves every p <= 2^kRescaleSlack, the bound the lazy rescale keeps,
@@ -637,7 +726,7 @@ struct Wave32 {
 #pragma unroll
                 for (int t = 0; t < 8; ++t)
                     pf[c][t] = (T)__builtin_amdgcn_exp2f(
-                        __builtin_fmaf(s[c >> 1][8 * (c & 1) + t], a.scale_log2, -m_run));
+                        __builtin_fmaf(s[c >> 1][8 * (c & 1) + t], to_log2, -m_run));
 #pragma unroll
                 for (int t = 0; t < 8; t += 2)
                     fsum = Dot2<T>::sum2(typename Dot2<T>::v2{pf[c][t], pf[c][t + 1]}, fsum);
@@ -647,15 +736,14 @@ struct Wave32 {
                 return;
             }
         }
-        const bool capped = MOD == MOD_GENERAL && a.softcap > 0.0f;  // uniform
         const float cap_hi = a.softcap * kLog2e, cap_m2 = -2.0f * a.softcap * kLog2e;
         if (raw) {
-            if (a.scale_log2 >= 0.0f) {
+            if (MOD == MOD_DENSE || a.scale_log2 >= 0.0f) {
 #pragma unroll
                 for (int sb = 0; sb < BN / 32; ++sb)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[sb][e]);
-                mx *= a.scale_log2;
+                mx *= to_log2;
             } else {
                 float mn = __builtin_huge_valf();
 #pragma unroll
@@ -674,7 +762,7 @@ struct Wave32 {
                 for (int e = 0; e < 16; ++e) mn = fminf(mn, s[sb][e]);
             mx = __builtin_fmaf(mn, cap_m2, cap_hi);  // -inf when every score is masked
         } else {
-            if (MOD == MOD_GENERAL) {
+            if (MOD != MOD_PLAIN) {
                 general_scores(k0);
             } else {
 #pragma unroll
@@ -707,7 +795,7 @@ struct Wave32 {
 #pragma unroll
                 for (int t = 0; t < 8; ++t)
                     pf[c][t] = (T)__builtin_amdgcn_exp2f(
-                        __builtin_fmaf(s[c >> 1][8 * (c & 1) + t], a.scale_log2, -m_use));
+                        __builtin_fmaf(s[c >> 1][8 * (c & 1) + t], to_log2, -m_use));
         } else if (capped) {
             const float c0 = cap_hi - m_use;
 #pragma unroll

@@ -186,6 +186,9 @@ hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipS
 hipError_t launch_key_groups(const FwdArgs& a, int dtype, int groups, hipStream_t s);
 // Keys of a staged tile: what one step of all groups covers.
 int key_group_keys(int kernel_dim, int groups);
+// 16-bit calls with a dense bias and no block mask, kernel head dims up to 128
+// (flash_bias.hip), on the score_mod kernel's tiling and plans.
+hipError_t launch_bias(const FwdArgs& a, int dtype, hipStream_t s);
 // Calls with a few query rows (decode_fwd.hip): plain scale, no mask.
 hipError_t launch_decode(const FwdArgs& a, int dtype, hipStream_t s);
 constexpr int kDecodeThreads = 512;
