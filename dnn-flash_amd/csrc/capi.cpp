@@ -264,7 +264,7 @@ void no_key_split(const ofh_attention_params* p, Resolved& r) {
     set_lds_list(p, r);
 }
 
-// 16-bit plain-scale calls that the planner would split over workgroups (few
+// 16-bit calls that the planner would split over workgroups (few
 // query tiles, so without a split CUs stay idle) run wavefront groups instead
 // where those are faster: no partial rows in memory and no merge launch, but
 // each staged K/V tile serves 1/groups of the query rows.
@@ -278,12 +278,18 @@ void no_key_split(const ofh_attention_params* p, Resolved& r) {
 // 74, H16 M500 N4000 36 / 54: from about 38 us (30 at kernel dim 96, 26 up to
 // 64) the chain outweighs what the merge costs. Causal pairs split in ranges
 // of their own lose less, hence their lower line (H128 N512 55 / 33, H32 N2048
-// 68 / 70). Few rows (one 128-row tile) leave groups without their gain (H64
+// 68 / 70). A score_mod makes both sides longer in like measure (ALiBi +
+// soft-cap D128 causal H8 N4096 76 / 74, H32 N1000 51 / 30; over 150 such shapes
+// the better count gains 1.5x), but a dense bias is staged through LDS by the
+// split plan's kernel and read by the lanes here, so its line is lower (shared
+// bias D64 non-causal H16 N1000 24 / 19, N1500 38 / 40, N2048 47 / 55). The
+// fewer the rows in all, the less a split has to merge (H32 M168 N2929 D128 32 /
+// 45, H2 N2500 29 / 32), hence the last factor. Few rows (one 128-row tile) leave groups without their gain (H64
 // M64 N1000 16 / 18), and grids of less than 32 128-row tiles keep the split,
 // on whose workspace and launch description their callers may rely.
 void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
-    if (p->dtype == OFH_DTYPE_F32 || p->max_key_splits != 0 || r.key_splits <= 1 || r.decode || r.general_mod ||
-        r.tile_list || r.kdim > 128 || p->query_tokens <= 128)
+    if (p->dtype == OFH_DTYPE_F32 || p->max_key_splits != 0 || r.key_splits <= 1 || r.decode || r.tile_list ||
+        r.kdim > 128 || p->query_tokens <= 128)
         return;
     const int64_t bh = (int64_t)p->batch * p->heads, M = (int64_t)p->query_tokens, N = (int64_t)p->key_tokens;
     if (bh * ((M + 127) / 128) < 32) return;
@@ -318,7 +324,10 @@ void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
         }
     }
     const float line[3] = {26.0f, 30.0f, 38.0f};
-    if (best_us > line[dim] * (r.pair_split ? 0.8f : 1.0f)) return;
+    if (best_us > line[dim] * (r.pair_split ? 0.8f : 1.0f) *
+                      (p->bias_kind == OFH_BIAS_DENSE ? 0.7f : 1.0f) * std::min(1.0f, (float)(bh * M) / 8192.0f))
+        return;
+    r.staged_bias = false;
     no_key_split(p, r);
     r.groups = best;
     r.paired = false;
@@ -393,8 +402,14 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     r.num_q_tiles = (int)((p->query_tokens + r.block_m - 1) / r.block_m);
     r.num_k_tiles = (int)((p->key_tokens + r.block_n - 1) / r.block_n);
     r.tile_list = p->mask_allowed != nullptr;
-    // (above 128 the K/V stages leave no room for the bias tiles in LDS)
-    r.staged_bias = p->dtype != OFH_DTYPE_F32 && p->bias_kind == OFH_BIAS_DENSE && !r.tile_list && r.kdim <= 128;
+    // (above 128 the K/V stages leave no room for the bias tiles in LDS; the
+    // kernel shares the score_mod kernel's plans, so this alignment rule moves
+    // no call's workspace)
+    if (p->dtype != OFH_DTYPE_F32 && p->bias_kind == OFH_BIAS_DENSE && !r.tile_list && r.kdim <= 128) {
+        int64_t bs[3];
+        dense_bias_strides(p, bs);
+        r.staged_bias = ofh::bias_can_be_staged(p->bias, (int64_t)p->key_tokens, bs[0], bs[1], bs[2]);
+    }
     // A few query rows (decoding), plain scale and no mask: the vector kernel
     // that streams K and V through registers. Planned as one 32-row query
     // block per head. (2^30: its key positions are 32-bit sums.)
@@ -1023,7 +1038,7 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
         // wavefront groups that split the keys inside a workgroup
         if (r.groups > 0) {
             pair_name = std::string("flash_fwd_keygroups_kernel<") + (p->dtype == OFH_DTYPE_BF16 ? "bf16," : "f16,") +
-                        std::to_string(r.kdim) + ",plain," + std::to_string(r.groups) + "groups>";
+                        std::to_string(r.kdim) + (r.general_mod ? ",mod," : ",plain,") + std::to_string(r.groups) + "groups>";
             name = pair_name.c_str();
         }
         // 16-bit causal pairs with a key split run the same tiling in a kernel of their own

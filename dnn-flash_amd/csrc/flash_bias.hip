@@ -13,9 +13,11 @@
 // the row-sum bound of Wave32::softmax.
 //
 // Measured (us, score_mod kernel -> this): fp16 B2 H16 N2048 D64, shared bias
-// 104.5 -> 67.2 (bias rows of no 16-byte alignment, N2047: 106.6 -> 93.8; a
-// bias per head, 537 MB of it: 141 -> 126, 4.3 TB/s), causal 78.7 -> 57.7; D32
-// B4 H16 N1024 41.8 -> 28.6; D128 H16 N4096 218 -> 178.
+// 104.5 -> 67.2 (a bias per head, 537 MB of it: 141 -> 126, 4.3 TB/s), causal 78.7
+// -> 57.7; D32 B4 H16 N1024 41.8 -> 28.6; D128 H16 N4096 218 -> 178. Rows that
+// are not 16-byte aligned would need four times the copies, 4 bytes per lane:
+// built and measured within 15 % of the score_mod kernel on either side (N2047
+// D64 107 -> 94, causal H96 N1767 D128 192 -> 225), so they stay there.
 
 #include "flash_wave32.h"
 #include "ofh_kernels.h"
@@ -31,7 +33,7 @@ constexpr int kBiasThreads = kBiasWaves * 64;
 // split evenly over the eight wavefronts (as in the score_mod kernel).
 constexpr int bias_steps(int D) { return D == 32 || D == 96 ? 2 : 1; }
 
-template <typename T, int D, bool SPLIT, bool VEC>
+template <typename T, int D, bool SPLIT>
 __device__ __forceinline__ void bias_qtile(const FwdArgs& a, unsigned char* smem, int bh, int qt, int split) {
     constexpr int BN = kBlockN16, SB = bias_steps(D);
     constexpr int BLOCK_M = kBiasWaves * kQueriesPerWave;
@@ -55,7 +57,7 @@ __device__ __forceinline__ void bias_qtile(const FwdArgs& a, unsigned char* smem
     }
     const int e1 = min(st1 * SB, (kend + BN - 1) / BN);  // compute steps [st0 SB, e1)
     w.copy_tile(st0, 0);
-    w.template copy_bias<VEC>(st0 * SB);
+    w.copy_bias(st0 * SB);
     wait_vm_loads();
     w.zero_tail(st0, 0);
     __syncthreads();
@@ -76,7 +78,7 @@ __device__ __forceinline__ void bias_qtile(const FwdArgs& a, unsigned char* smem
                 bias_pending = false;
                 if (e + 1 < e1 && w.tile_active(e + 1)) {
                     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the softmax has read its bias
-                    w.template copy_bias<VEC>(e + 1);
+                    w.copy_bias(e + 1);
                     bias_pending = true;
                 }
                 w.pv(stage, j);
@@ -84,7 +86,7 @@ __device__ __forceinline__ void bias_qtile(const FwdArgs& a, unsigned char* smem
         }
         // the K/V copies have landed; the next step's bias may still be in flight
         if (!bias_pending) wait_vm_loads();
-        else wait_vm<VEC ? 8 : 32>();
+        else wait_vm<8>();
         if (st + 1 < st1) w.zero_tail(st + 1, nstage);
         __syncthreads();
     }
@@ -93,7 +95,7 @@ __device__ __forceinline__ void bias_qtile(const FwdArgs& a, unsigned char* smem
 
 // MODE 0: a query tile (and key split) per workgroup; 1: causal pairs of query
 // tiles; 2: causal pairs, each tile split in ranges of its own length.
-template <typename T, int D, int MODE, bool VEC>
+template <typename T, int D, int MODE>
 __global__ __launch_bounds__(kBiasThreads, 1) void flash_fwd_bias_kernel(FwdArgs a) {
     using W = Wave32<T, D, MOD_DENSE, false, kBiasThreads, kBlockN16, bias_steps(D)>;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * W::L::STAGE + kBiasWaves * W::BIAS_BYTES];
@@ -102,37 +104,37 @@ __global__ __launch_bounds__(kBiasThreads, 1) void flash_fwd_bias_kernel(FwdArgs
         const int tiles = a.B * a.H * a.num_q_tiles;
         const int split = (int)blockIdx.x / tiles;
         map_work((int)blockIdx.x - split * tiles, a.B * a.H, a.num_q_tiles, a.causal, bh, qts[0]);
-        bias_qtile<T, D, true, VEC>(a, smem, bh, qts[0], split);
+        bias_qtile<T, D, true>(a, smem, bh, qts[0], split);
     } else {
         const int pairs = a.B * a.H * ((a.num_q_tiles + 1) / 2);
         const int split = MODE == 2 ? (int)blockIdx.x / pairs : 0;
         map_work_pair((int)blockIdx.x - split * pairs, a.B * a.H, a.num_q_tiles, bh, qts[0], qts[1]);
-        bias_qtile<T, D, MODE == 2, VEC>(a, smem, bh, qts[0], split);
+        bias_qtile<T, D, MODE == 2>(a, smem, bh, qts[0], split);
         if (qts[1] >= 0) {
             __syncthreads();  // LDS stages are reused
-            bias_qtile<T, D, MODE == 2, VEC>(a, smem, bh, qts[1], split);
+            bias_qtile<T, D, MODE == 2>(a, smem, bh, qts[1], split);
         }
     }
 }
 
-template <typename T, int D, bool VEC>
+template <typename T, int D>
 hipError_t launch_bias_d(const FwdArgs& a, hipStream_t s) {
     const bool paired = a.pair_split != 0 || (a.causal && a.num_splits == 1);
     const int64_t tiles = paired ? (a.num_q_tiles + 1) / 2 : a.num_q_tiles;
     const dim3 grid((unsigned)((int64_t)a.B * a.H * tiles * a.num_splits)), block(kBiasThreads);
-    if (a.pair_split) hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 2, VEC>), grid, block, 0, s, a);
-    else if (paired) hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 1, VEC>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 0, VEC>), grid, block, 0, s, a);
+    if (a.pair_split) hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 2>), grid, block, 0, s, a);
+    else if (paired) hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 1>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((flash_fwd_bias_kernel<T, D, 0>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-template <typename T, bool VEC>
+template <typename T>
 hipError_t launch_bias_t(const FwdArgs& a, int kd, hipStream_t s) {
     switch (kd) {
-        case 32: return launch_bias_d<T, 32, VEC>(a, s);
-        case 64: return launch_bias_d<T, 64, VEC>(a, s);
-        case 96: return launch_bias_d<T, 96, VEC>(a, s);
-        case 128: return launch_bias_d<T, 128, VEC>(a, s);
+        case 32: return launch_bias_d<T, 32>(a, s);
+        case 64: return launch_bias_d<T, 64>(a, s);
+        case 96: return launch_bias_d<T, 96>(a, s);
+        case 128: return launch_bias_d<T, 128>(a, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -141,13 +143,10 @@ hipError_t launch_bias_t(const FwdArgs& a, int kd, hipStream_t s) {
 
 hipError_t launch_bias(const FwdArgs& a, int dtype, hipStream_t s) {
     const int kd = flash_mfma_kernel_dim(dtype, a.D, a.Dv);
-    if (a.mask != nullptr || a.bias_kind != BIAS_DENSE || a.split_bm != kBiasWaves * kQueriesPerWave)
+    if (a.mask != nullptr || a.bias_kind != BIAS_DENSE || a.split_bm != kBiasWaves * kQueriesPerWave ||
+        !bias_can_be_staged(a.bias, a.N, a.bias_sb, a.bias_sh, a.bias_sm))
         return hipErrorInvalidValue;
-    // 16-byte copies of bias rows: aligned rows of whole chunks, 32-bit offsets within 32 rows
-    const bool vec = (uintptr_t)a.bias % 16 == 0 && a.N % 4 == 0 && a.bias_sb % 4 == 0 && a.bias_sh % 4 == 0 &&
-                  a.bias_sm % 4 == 0 && a.bias_sm < (1 << 24);
-    if (dtype == DT_F16) return vec ? launch_bias_t<_Float16, true>(a, kd, s) : launch_bias_t<_Float16, false>(a, kd, s);
-    return vec ? launch_bias_t<__bf16, true>(a, kd, s) : launch_bias_t<__bf16, false>(a, kd, s);
+    return dtype == DT_F16 ? launch_bias_t<_Float16>(a, kd, s) : launch_bias_t<__bf16>(a, kd, s);
 }
 
 }  // namespace ofh

@@ -15,7 +15,10 @@
 // softmax one after the other) times the longest chain. Measured (us, split
 // 256-row tiles -> this): bf16 causal H32 D128 N512 25.8 -> 13.3, N1000 42.7 ->
 // 23.2, N1500 54 -> 45; H128 N512 54.6 -> 32.7; D64 H16 N1500 non-causal 28.7 ->
-// 21.0. Asking for a head's K and V rows ahead (one load per line at the start)
+// 21.0. With a score_mod: ALiBi + soft-cap H32 D128 N512 26.2 -> 15.1 causal,
+// N1000 44.5 -> 30.8 non-causal; shared bias H16 D64 N1000 30.7 -> 18.8. (A dense
+// bias is read by the lanes here: its LDS tiles would not fit beside four
+// groups' keys.) Asking for a head's K and V rows ahead (one load per line at the start)
 // gained 0-3 % up to N1500, so it is not done.
 
 #include "flash_wave32.h"
@@ -117,13 +120,18 @@ __global__ __launch_bounds__(kGroupThreads, 1) void flash_fwd_keygroups_kernel(F
     }
 }
 
-template <typename T, int D>
-hipError_t launch_groups(const FwdArgs& a, int groups, hipStream_t s) {
+template <typename T, int D, int MOD>
+hipError_t launch_groups_mod(const FwdArgs& a, int groups, hipStream_t s) {
     const dim3 grid((unsigned)((int64_t)a.B * a.H * a.num_q_tiles)), block(kGroupThreads);
-    if (groups == 2) hipLaunchKernelGGL((flash_fwd_keygroups_kernel<T, D, 2, MOD_PLAIN>), grid, block, 0, s, a);
-    else if (groups == 4) hipLaunchKernelGGL((flash_fwd_keygroups_kernel<T, D, 4, MOD_PLAIN>), grid, block, 0, s, a);
+    if (groups == 2) hipLaunchKernelGGL((flash_fwd_keygroups_kernel<T, D, 2, MOD>), grid, block, 0, s, a);
+    else if (groups == 4) hipLaunchKernelGGL((flash_fwd_keygroups_kernel<T, D, 4, MOD>), grid, block, 0, s, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
+}
+template <typename T, int D>
+hipError_t launch_groups(const FwdArgs& a, int groups, hipStream_t s) {
+    return a.bias_kind != BIAS_NONE || a.softcap > 0.0f ? launch_groups_mod<T, D, MOD_GENERAL>(a, groups, s)
+                                                        : launch_groups_mod<T, D, MOD_PLAIN>(a, groups, s);
 }
 
 }  // namespace

@@ -158,19 +158,12 @@ __device__ __forceinline__ void dma16(const void* g, unsigned lds) {
                  : "=&s"(save) : "v"(g), "s"(lds) : "memory");
 }
 
-// The same from a wave-uniform base plus a per-lane byte offset, 16 or 4 bytes
-// per lane (lane L writes lds + 16 L or lds + 4 L).
+// The same from a wave-uniform base plus a per-lane byte offset.
 __device__ __forceinline__ void dma16s(const void* base, unsigned off, unsigned lds) {
     unsigned save;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                  : "=&s"(save) : "v"(off), "s"(base), "s"(lds) : "memory");
 }
-__device__ __forceinline__ void dma4(const void* base, unsigned off, unsigned lds) {
-    unsigned save;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(save) : "v"(off), "s"(base), "s"(lds) : "memory");
-}
-
 // K and V tiles in LDS: row-major [key][d], unpadded (each global -> LDS
 // copy instruction writes 1 KB of consecutive LDS). Chunk c (16 bytes) of row
 // r sits at position c ^ kswz(r) (K) or c ^ vswz(r) (V), which keeps both
@@ -467,11 +460,10 @@ struct Wave32 {
     // global -> LDS (asynchronous) into 32 rows of BN floats of its own at
     // bias_lds. 16-byte chunk c of row r sits at chunk c ^ (r & 15): a read
     // takes one chunk of 16 rows, 256 bytes apart. Rows past M and keys past N
-    // repeat the last one (their scores are masked or never stored). VEC:
-    // 16-byte aligned rows and N a multiple of 4, eight copies of four rows;
-    // else 32 of one row, 4 bytes per lane.
+    // repeat the last one (their scores are masked or never stored). Eight copies
+    // of four rows each; rows are 16-byte aligned, N is a multiple of 4 and the
+    // row stride at most 2^24 (bias_can_be_staged).
     static constexpr int BIAS_BYTES = 32 * BN * 4;  // per wavefront
-    template <bool VEC>
     __device__ __forceinline__ void copy_bias(int e) {
         static_assert(BN == 64, "a bias row is 16 chunks");
         const int k0 = e * BN;
@@ -481,7 +473,7 @@ struct Wave32 {
         // formed here each time instead of kept in registers: at D = 128 those spill)
         int lane = tid & 63;
         asm volatile("" : "+v"(lane));
-        if (VEC && k0 + BN <= a.N && qw0 + kQueriesPerWave <= a.M) {
+        if (k0 + BN <= a.N && qw0 + kQueriesPerWave <= a.M) {
             // copy u: rows 4u + lane / 16, chunk (lane % 16) ^ (lane / 16) ^ 4 (u % 4)
             const unsigned roff = 4u * (unsigned)((lane >> 4) * (int)a.bias_sm);
             const unsigned c0 = 16u * (unsigned)((lane & 15) ^ (lane >> 4));
@@ -490,22 +482,13 @@ struct Wave32 {
                 dma16s(base, (c0 ^ (64u * (u & 3))) + roff, lds0 + 1024 * u);
                 base += 4 * a.bias_sm;
             }
-        } else if constexpr (VEC) {
+        } else {
             const int last_row = max(0, a.M - 1 - qw0), last = a.N - 4 - k0;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const int row = 4 * u + (lane >> 4);
                 const int key = min(4 * ((lane & 15) ^ (row & 15)), last);
                 dma16s(base, 4u * (unsigned)(min(row, last_row) * (int)a.bias_sm + key), lds0 + 1024 * u);
-            }
-        } else {
-            const unsigned off0 = 4u * (unsigned)lane, last = 4u * (unsigned)(a.N - 1 - k0);
-            int rows = a.M - qw0;  // likewise: 32 row conditions kept would spill scalar registers
-            asm volatile("" : "+s"(rows));
-#pragma unroll
-            for (int u = 0; u < 32; ++u) {
-                dma4(base, min(off0 ^ (16u * (u & 15)), last), lds0 + 256 * u);
-                base += u + 1 < rows ? a.bias_sm : 0;
             }
         }
     }

@@ -181,13 +181,18 @@ struct QkScoreArgs {
 // Launchers; each returns the hipError_t of the launch.
 hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipStream_t s);
 // 16-bit calls whose eight wavefronts split the keys of 256 / groups query rows
-// (flash_keygroups.hip), groups = 2 or 4; kernel head dims up to 128, plain
-// scale, no block mask, no key split over workgroups.
+// (flash_keygroups.hip), groups = 2 or 4; kernel head dims up to 128, no block
+// mask, no key split over workgroups.
 hipError_t launch_key_groups(const FwdArgs& a, int dtype, int groups, hipStream_t s);
 // Keys of a staged tile: what one step of all groups covers.
 int key_group_keys(int kernel_dim, int groups);
 // 16-bit calls with a dense bias and no block mask, kernel head dims up to 128
-// (flash_bias.hip), on the score_mod kernel's tiling and plans.
+// (flash_bias.hip), on the score_mod kernel's tiling and plans, where the bias
+// can be copied 16 bytes at a time: aligned rows of whole chunks, and 32-bit
+// offsets within 32 rows.
+inline bool bias_can_be_staged(const float* bias, int64_t N, int64_t sb, int64_t sh, int64_t sm) {
+    return ((uintptr_t)bias & 15) == 0 && ((N | sb | sh | sm) & 3) == 0 && sm <= (1 << 24);
+}
 hipError_t launch_bias(const FwdArgs& a, int dtype, hipStream_t s);
 // Calls with a few query rows (decode_fwd.hip): plain scale, no mask.
 hipError_t launch_decode(const FwdArgs& a, int dtype, hipStream_t s);

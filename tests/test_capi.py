@@ -378,7 +378,7 @@ def test_kernel_choice(ofh):
 
 
 def test_key_group_choice(ofh):
-    """Wavefront groups replace the key split over workgroups of 16-bit plain
+    """Wavefront groups replace the key split over workgroups of 16-bit
     calls with at least 32 query tiles of 128 rows and short chains; every
     other call keeps its plan."""
     F = ofh
@@ -392,13 +392,16 @@ def test_key_group_choice(ofh):
     assert name(1, 8, 1000, 1000, 64) == groups + "64,plain,4groups>"
     assert name(2, 8, 1000, 1000, 80) == groups + "96,plain,4groups>"
     assert name(1, 128, 512, 512, 128, causal=True) == groups + "128,plain,2groups>"  # pairs that would split
+    assert name(1, 32, 1000, 1000, 128, causal=True, softcap=5.0) == groups + "128,mod,2groups>"
+    dense = dict(bias_kind=F.BIAS_DENSE, bias=16)
+    assert name(1, 16, 1000, 1000, 64, **dense) == groups + "64,mod,4groups>"
+    assert name(1, 16, 1500, 1500, 64, **dense) == "flash_fwd_bias_kernel<bf16,64>"
     p = F.make_params(1, 32, 1000, 1000, 128, dtype=F.DTYPE_BF16, causal=True)
     info = F.launch_info(p)
     assert info.block_m == 128 and info.block_n == 128 and info.threads == 512 and info.workgroups == 32 * 8
     assert info.key_splits == 1 and F.workspace_bytes(p) == 0
     for other in [name(1, 32, 1000, 1000, 128, causal=True, max_key_splits=1),
                   name(1, 32, 1000, 1000, 128, causal=True, max_key_splits=2),
-                  name(1, 32, 1000, 1000, 128, causal=True, softcap=5.0),
                   name(1, 32, 1000, 1000, 160, causal=True),
                   name(1, 10, 300, 300, 128),         # 30 tiles of 128 rows
                   name(1, 64, 128, 1000, 128),        # one tile of rows per head

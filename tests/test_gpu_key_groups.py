@@ -8,7 +8,7 @@ import math
 import numpy as np
 import pytest
 
-from gpu_helpers import THREADS, assert_bars, make_inputs, norm_error
+from gpu_helpers import THREADS, alibi_slopes, assert_bars, make_inputs, norm_error
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +56,33 @@ def test_key_groups(ofh, dt, D, Dv, shapes):
         assert_bars(err, dt, f"{dt} {name} M{M} N{N} causal={causal}")
         low = F.attention_fwd(*dev, causal=causal)
         assert torch.equal(low, torch.from_numpy(out).cuda().to(low.dtype))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("D,Dv,H,M,N,causal,mod", [
+    (64, 64, 12, 300, 333, False, "alibi+cap"), (128, 128, 32, 500, 500, True, "alibi"),
+    (96, 96, 32, 700, 700, True, "cap"), (64, 64, 16, 777, 777, False, "dense"),
+    (128, 72, 16, 513, 300, True, "dense+cap"), (32, 32, 64, 129, 200, False, "dense")])
+def test_key_groups_score_mod(ofh, dt, D, Dv, H, M, N, causal, mod):
+    """The same kernel with every kind of score modification."""
+    F = ofh
+    cap = 20.0 if "cap" in mod else 0.0
+    kind = F.BIAS_ALIBI if "alibi" in mod else F.BIAS_DENSE if "dense" in mod else F.BIAS_NONE
+    p = F.make_params(1, H, M, N, D, Dv, dtype=DTYPE[dt], causal=causal, softcap=cap, bias_kind=kind,
+                      alibi_slopes=16 if kind == F.BIAS_ALIBI else None, bias=16 if kind == F.BIAS_DENSE else None)
+    name = F.launch_info(p).kernel_name.decode()
+    assert name.startswith("flash_fwd_keygroups_kernel<") and ",mod," in name, name
+    dev, host = make_inputs(dt, 1, H, M, N, D, Dv, seed=M)
+    slopes = alibi_slopes(H) if kind == F.BIAS_ALIBI else None
+    bias = O.normal(5, (M, N), std=2.0) if kind == F.BIAS_DENSE else None
+    kw = {} if slopes is None else {"alibi_slopes": torch.from_numpy(slopes).cuda()}
+    if bias is not None:
+        kw["bias"] = torch.from_numpy(bias).cuda()
+    out = F.attention_fwd(*dev, causal=causal, softcap=cap, out_dtype=torch.float32, **kw).cpu().numpy()
+    prob = O.Problem(1, H, M, N, D, Dv, scale=1.0 / math.sqrt(D), causal=causal, alibi_slopes=slopes,
+                     dense_bias=bias, softcap=cap)
+    heads = np.array([0, H // 2, H - 1], dtype=np.uint64)
+    ref = O.standard_attention_rows(*host, prob, np.repeat(heads, M), np.tile(np.arange(M, dtype=np.uint64), 3),
+                                    threads=THREADS).reshape(3, M, Dv)
+    err, _ = norm_error(out.reshape(H, M, Dv)[heads.astype(int)], ref)
+    assert_bars(err, dt, f"{dt} {name} M{M} N{N} causal={causal} {mod}")
