@@ -5,8 +5,8 @@
 // 48-69 post-ops after matmul_tile_strided_inplace, whose reference kernel
 // sums over k sequentially in fp32, src/onednn_flash/tile_kernel.cpp:49-86).
 // Every product and every partial sum is rounded once, in the same order, so
-// fp32 results are bit-identical to the reference. 32x32 output blocks per
-// workgroup; Q and K^T chunks of 32 along k are staged through LDS as fp32.
+// fp32 results are bit-identical to the reference. 32x32 or 64x64 output blocks
+// per workgroup; Q and K^T chunks of 32 along k are staged through LDS as fp32.
 //
 // For bf16/fp16 inputs a matrix-core variant computes the same scores with
 // v_mfma_f32_32x32x16_{bf16,f16}: the products are exact in fp32 and only the
@@ -20,68 +20,151 @@
 namespace ofh {
 namespace {
 
-constexpr int kQkTile = 32;
 constexpr int64_t kMaxGridZ = 65535;   // tiles per launch (grid z)
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 
-template <typename T>
+// Exact scores. A workgroup of 16 x 16 threads forms a block of 16 PT x 16 PT
+// scores, PT x PT per thread; chunks of 32 along k of its Q and K rows are
+// staged in LDS as fp32, k-major, so that a wavefront reads consecutive K
+// elements and broadcasts Q. The next chunk is on its way through registers
+// while this one is multiplied, and the LDS is double-buffered (one barrier per
+// chunk).
+//
+// What bounds it: the vector ALU, two instructions per multiply-add because
+// product and sum are rounded separately, and the LDS: per k a thread reads 2 PT
+// floats for PT^2 multiply-adds. Measured, fp32 32 tiles 1024^2 x 128: 343 us
+// with 4 scores of one column per thread (a read per multiply-add, 64-bit index
+// arithmetic per load), 192 us with PT = 4 (45 TFLOP/s of useful work).
+template <typename T, int PT>
 __global__ __launch_bounds__(256) void qk_score_kernel(QkScoreArgs a) {
     // Products, sums, scale and bias are each rounded: no contraction to FMA.
 #pragma clang fp contract(off)
-    __shared__ float qs[kQkTile][kQkTile + 1];   // [row i][kk]
-    __shared__ float ks[kQkTile][kQkTile + 1];   // [kk][col j]
+    constexpr int BT = 16 * PT;      // scores per block side
+    constexpr int BK = 32;           // k per chunk
+    constexpr int STR = BT + 4;      // floats per k row of a staged chunk
+    constexpr int LOADS = BT * BK / 256;
+    constexpr int GW = PT < 4 ? PT : 4, NG = PT / GW;  // a thread's rows (columns): NG groups of GW, 16 GW apart
+    typedef float vec __attribute__((ext_vector_type(GW)));
+    __shared__ __attribute__((aligned(16))) float qs[2][BK * STR], ks[2][BK * STR];
     const int tid = threadIdx.x;
-    const int tx = tid & 31, ty = tid >> 5;      // column, row group (8 groups of 4 rows)
+    const int tx = tid & 15, ty = tid >> 4;
     const int64_t bt = blockIdx.z;
-    const int64_t i0 = (int64_t)blockIdx.y * kQkTile, j0 = (int64_t)blockIdx.x * kQkTile;
-    const T* q = (const T*)a.q + bt * a.a_sb;
-    const T* k = (const T*)a.k + bt * a.b_sb;
-    const bool q_k_fast = a.a_sk <= a.a_sm, k_k_fast = a.b_sk <= a.b_sn;
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t k0 = 0; k0 < a.K; k0 += kQkTile) {
-        // Stage both chunks, zero outside the tile. Lanes walk whichever axis
-        // has the smaller stride so that row-major Q [m,k] and K [n,k] (both
-        // contiguous along k) are read with unit stride.
+    const int64_t i0 = (int64_t)blockIdx.y * BT, j0 = (int64_t)blockIdx.x * BT;
+    // Lanes walk whichever axis has the smaller stride (row-major Q [m,k] and
+    // K [n,k] are both contiguous along k): load u of a thread is element
+    // (row r0 + u rs, k kk0 + u kks) of the chunk. Elements outside the tile are 0.
+    struct Side {
+        int r0, rs, kk0, kks, rows, lds, lds_step;
+        const T* p;
+        int64_t step, chunk;
+    };
+    auto side = [&](const T* base, int64_t sr, int64_t sk, int64_t row0, int64_t rows) {
+        const bool k_fast = sk <= sr;  // uniform
+        Side d;
+        d.r0 = k_fast ? tid / BK : tid % BT;
+        d.rs = k_fast ? 256 / BK : (256 % BT);  // (BT divides 256 or 256 BT; k_fast false: rows repeat)
+        d.kk0 = k_fast ? tid % BK : tid / BT;
+        d.kks = k_fast ? 0 : 256 / BT;
+        d.rows = (int)min((int64_t)BT, rows - row0);
+        d.lds = d.kk0 * STR + d.r0;
+        d.lds_step = d.kks * STR + d.rs;
+        d.p = base + (row0 + d.r0) * sr + d.kk0 * sk;
+        d.step = d.rs * sr + d.kks * sk;
+        d.chunk = BK * sk;
+        return d;
+    };
+    static_assert(256 % BT == 0 && 256 % BK == 0, "a load covers whole rows or whole k steps");
+    Side sq = side((const T*)a.q + bt * a.a_sb, a.a_sm, a.a_sk, i0, a.M);
+    Side sk = side((const T*)a.k + bt * a.b_sb, a.b_sn, a.b_sk, j0, a.N);
+    float rq[LOADS], rk[LOADS];
+    auto load = [&](Side& d, float (&r)[LOADS], int kleft) {  // kleft: k elements from this chunk on
+        const T* p = d.p;
+        if (d.rows == BT && kleft >= BK) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int r = ty + 8 * u;
-            if (q_k_fast) {
-                const int64_t qi = i0 + r, qk = k0 + tx;
-                qs[r][tx] = (qi < a.M && qk < a.K) ? to_f32(q[qi * a.a_sm + qk * a.a_sk]) : 0.0f;
-            } else {
-                const int64_t qi = i0 + tx, qk = k0 + r;
-                qs[tx][r] = (qi < a.M && qk < a.K) ? to_f32(q[qi * a.a_sm + qk * a.a_sk]) : 0.0f;
+            for (int u = 0; u < LOADS; ++u) r[u] = to_f32(p[u * d.step]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < LOADS; ++u)
+                r[u] = d.r0 + u * d.rs < d.rows && d.kk0 + u * d.kks < kleft ? to_f32(p[u * d.step]) : 0.0f;
+        }
+        d.p += d.chunk;
+    };
+    auto put = [&](const Side& d, const float (&r)[LOADS], float* lds) {
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) lds[d.lds + u * d.lds_step] = r[u];
+    };
+    float acc[PT][PT];
+#pragma unroll
+    for (int x = 0; x < PT; ++x)
+#pragma unroll
+        for (int y = 0; y < PT; ++y) acc[x][y] = 0.0f;
+    const int K = (int)a.K;
+    load(sq, rq, K);
+    load(sk, rk, K);
+    put(sq, rq, qs[0]);
+    put(sk, rk, ks[0]);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += BK) {
+        const bool more = K - k0 > BK;
+        if (more) {
+            load(sq, rq, K - k0 - BK);
+            load(sk, rk, K - k0 - BK);
+        }
+        const float *ql = &qs[buf][GW * ty], *kl = &ks[buf][GW * tx];
+        auto step = [&](int t) {
+#pragma clang fp contract(off)  // (a lambda's body does not take the function's pragma)
+            vec qv[NG], kv[NG];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                qv[g] = *(const vec*)(ql + t * STR + 16 * GW * g);
+                kv[g] = *(const vec*)(kl + t * STR + 16 * GW * g);
             }
-            if (k_k_fast) {
-                const int64_t kk = k0 + tx, kj = j0 + r;
-                ks[tx][r] = (kk < a.K && kj < a.N) ? to_f32(k[kk * a.b_sk + kj * a.b_sn]) : 0.0f;
-            } else {
-                const int64_t kk = k0 + r, kj = j0 + tx;
-                ks[r][tx] = (kk < a.K && kj < a.N) ? to_f32(k[kk * a.b_sk + kj * a.b_sn]) : 0.0f;
-            }
+#pragma unroll
+            for (int x = 0; x < PT; ++x)
+#pragma unroll
+                for (int y = 0; y < PT; ++y) acc[x][y] = acc[x][y] + qv[x / GW][x % GW] * kv[y / GW][y % GW];
+        };
+        if (K - k0 >= BK) {
+#pragma unroll 8
+            for (int t = 0; t < BK; ++t) step(t);
+        } else {
+            for (int t = 0; t < K - k0; ++t) step(t);
+        }
+        if (more) {
+            put(sq, rq, qs[buf ^ 1]);
+            put(sk, rk, ks[buf ^ 1]);
         }
         __syncthreads();
-        const int kn = (int)min((int64_t)kQkTile, a.K - k0);
-        for (int t = 0; t < kn; ++t) {
-            const float b = ks[t][tx];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc[u] = acc[u] + qs[ty + 8 * u][t] * b;
-        }
-        __syncthreads();
+        buf ^= 1;
     }
-    const int64_t j = j0 + tx;
-    if (j >= a.N) return;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int64_t i = i0 + ty + 8 * u;
+    for (int x = 0; x < PT; ++x) {
+        const int64_t i = i0 + 16 * GW * (x / GW) + GW * ty + x % GW;
         if (i >= a.M) continue;
-        float v = acc[u];
-        if (a.has_scale) v = v * a.scale;
-        if (a.bias != nullptr) v = v + a.bias[bt * a.bias_sb + i * a.bias_sm + j * a.bias_sn];
-        if (a.softcap > 0.0f) v = a.softcap * tanhf(v / a.softcap);
-        a.c[bt * a.c_sb + i * a.c_sm + j * a.c_sn] = v;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int64_t j = j0 + 16 * GW * g + GW * tx;
+            vec v;
+#pragma unroll
+            for (int e = 0; e < GW; ++e) {
+                float w = acc[x][GW * g + e];
+                if (a.has_scale) w = w * a.scale;
+                if (a.bias != nullptr && j + e < a.N) w = w + a.bias[bt * a.bias_sb + i * a.bias_sm + (j + e) * a.bias_sn];
+                if (a.softcap > 0.0f) w = a.softcap * tanhf(w / a.softcap);
+                v[e] = w;
+            }
+            float* c = a.c + bt * a.c_sb + i * a.c_sm + j * a.c_sn;
+            if (a.vec4 && j + GW <= a.N) {
+                *(vec*)c = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < GW; ++e)
+                    if (j + e < a.N) c[e * a.c_sn] = v[e];
+            }
+        }
     }
 }
 
@@ -521,6 +604,21 @@ hipError_t launch_qk_score_mfma(const QkScoreArgs& a, int dtype, hipStream_t s) 
     return hipSuccess;
 }
 
+namespace {
+template <int PT>
+hipError_t launch_qk_exact(const QkScoreArgs& x, int dtype, hipStream_t s) {
+    const dim3 grid((unsigned)((x.N + 16 * PT - 1) / (16 * PT)), (unsigned)((x.M + 16 * PT - 1) / (16 * PT)),
+                    (unsigned)x.batch);
+    switch (dtype) {
+        case DT_F32: hipLaunchKernelGGL((qk_score_kernel<float, PT>), grid, dim3(256), 0, s, x); break;
+        case DT_BF16: hipLaunchKernelGGL((qk_score_kernel<__bf16, PT>), grid, dim3(256), 0, s, x); break;
+        case DT_F16: hipLaunchKernelGGL((qk_score_kernel<_Float16, PT>), grid, dim3(256), 0, s, x); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_qk_score(const QkScoreArgs& a, int dtype, hipStream_t s) {
     if (a.batch <= 0 || a.M <= 0 || a.N <= 0 || a.K <= 0) return hipSuccess;
     const size_t esz = dtype == DT_F32 ? 4 : 2;
@@ -531,15 +629,14 @@ hipError_t launch_qk_score(const QkScoreArgs& a, int dtype, hipStream_t s) {
         x.k = (const char*)a.k + b0 * a.b_sb * esz;
         x.c = a.c + b0 * a.c_sb;
         if (a.bias != nullptr) x.bias = a.bias + b0 * a.bias_sb;
-        const dim3 grid((unsigned)((a.N + kQkTile - 1) / kQkTile),
-                        (unsigned)((a.M + kQkTile - 1) / kQkTile), (unsigned)x.batch);
-        switch (dtype) {
-            case DT_F32: hipLaunchKernelGGL(qk_score_kernel<float>, grid, dim3(256), 0, s, x); break;
-            case DT_BF16: hipLaunchKernelGGL(qk_score_kernel<__bf16>, grid, dim3(256), 0, s, x); break;
-            case DT_F16: hipLaunchKernelGGL(qk_score_kernel<_Float16>, grid, dim3(256), 0, s, x); break;
-            default: return hipErrorInvalidValue;
-        }
-        const hipError_t e = hipGetLastError();
+        x.vec4 = a.c_sn == 1 && a.c_sm % 4 == 0 && a.c_sb % 4 == 0 && (reinterpret_cast<uintptr_t>(a.c) & 15u) == 0;
+        // 64x64 blocks where they give every CU three, 32x32 below (us, 32x32 /
+        // 64x64: 16 tiles 512^2 x 64, 1024 blocks, 24.4 / 20.3; 8 tiles 333 x 777 x
+        // 100, 624 blocks, 24.0 / 25.4; 20 tiles 250 x 430 x 64, 560 blocks, 16.4 /
+        // 18.6; 4 tiles 128^2 x 64, 16 blocks, 5.6 / 10.2). 128x128 blocks gained
+        // 1 % at 32 tiles 1024^2 x 128 and lost 35 % at 8 tiles 1100^2 x 96.
+        const int64_t blocks64 = x.batch * ((x.M + 63) / 64) * ((x.N + 63) / 64);
+        const hipError_t e = blocks64 >= 3 * kComputeUnits ? launch_qk_exact<4>(x, dtype, s) : launch_qk_exact<2>(x, dtype, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -92,6 +92,24 @@ def test_exact_kernel_bit_exact(ofh, dt, shape):
         np.testing.assert_array_equal(_bits(got.cpu().numpy()), _bits(want))
 
 
+@pytest.mark.parametrize("dt", ["f32", "f16"])
+@pytest.mark.parametrize("T,M,N,K", [(200, 65, 129, 33), (1100, 63, 40, 5), (3, 65, 129, 33), (2, 31, 33, 31)])
+def test_exact_kernel_block_edges(ofh, dt, T, M, N, K):
+    """Both block sizes of the exact kernel (64x64 from 768 blocks up) past their
+    row, column and k-chunk edges, with either axis of Q and K contiguous: bit
+    for bit the oracle's."""
+    rng = np.random.default_rng(T + K)
+    tq, uq = to_device(rng.standard_normal((T, M, K), dtype=np.float32), dt)
+    tk, uk = to_device(rng.standard_normal((T, N, K), dtype=np.float32), dt)
+    want = O.qk_score_tile(uq, uk, scale=0.3)
+    for flip_q in (False, True):
+        for flip_k in (False, True):
+            q = tq.transpose(1, 2).contiguous().transpose(1, 2) if flip_q else tq
+            k = tk.transpose(1, 2).contiguous().transpose(1, 2) if flip_k else tk
+            got = _run(ofh, q, k, scale=0.3, algorithm=ofh.QK_EXACT)
+            np.testing.assert_array_equal(_bits(got.cpu().numpy()), _bits(want))
+
+
 def test_exact_kernel_strided_views(ofh):
     rng = np.random.default_rng(11)
     big_q = rng.standard_normal((3, 50, 90), dtype=np.float32)
