@@ -230,6 +230,7 @@ __device__ __forceinline__ void dma16(const void* src, qk_lds_u8* dst) {
 __device__ __forceinline__ qk_u32x4 lds_read16(const qk_lds_u8* p) { return *(const qk_lds_u32x4*)p; }
 typedef float qk_f32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) qk_f32x4 qk_lds_f32x4;
+typedef __attribute__((address_space(3))) float qk_lds_f32;
 __device__ __forceinline__ void lds_write_f4(qk_lds_u8* p, qk_f32x4 v) { *(qk_lds_f32x4*)p = v; }
 __device__ __forceinline__ qk_f32x4 lds_read_f4(const qk_lds_u8* p) { return *(const qk_lds_f32x4*)p; }
 
@@ -362,8 +363,10 @@ __global__ __launch_bounds__(256) void qk_score_mfma_kernel(QkScoreArgs a) {
     }
 }
 
-// Score rows without a bias or soft-cap, K <= 128 (scores only need the scale):
-// one workgroup per 128-row query block and run of `tpw` 128-key blocks.
+// Post-operations of a row kernel instantiation (the scale is a run-time choice).
+enum QkPost { QK_POST_NONE = 0, QK_POST_BIAS = 1, QK_POST_CAP = 2, QK_POST_BIAS_CAP = 3 };
+
+// Score rows, K <= 128: one workgroup per 128-row query block and run of `tpw` 128-key blocks.
 // The query block's MFMA fragments stay in registers for the whole run; K
 // block t+1 is copied global -> LDS into the second buffer while block t is
 // multiplied and written, and the buffer block t was read from then stages
@@ -375,6 +378,17 @@ __global__ __launch_bounds__(256) void qk_score_mfma_kernel(QkScoreArgs a) {
 // takes a contiguous range of query blocks, i.e. reads the Q and K of a few
 // heads only. Same products and summation order as qk_score_mfma_kernel, so
 // the scores are bit-identical. CH = 16-byte chunks per K row in LDS (K <= 8 CH).
+//
+// A block's bias is requested into registers (32 per lane: one epilogue pass)
+// before its products, and the second pass's behind the first one's stores; read
+// in the epilogue it stood between each row's LDS read and its store. VEC: scores and bias are read and written as 16
+// lanes x 16 bytes per row (aligned rows, N a multiple of 4); else as 64 lanes x
+// 4 bytes, whole 256-byte row pieces as well. Measured (us, one-block kernel ->
+// this): bf16 32 tiles 2048^2 x 128 with a shared bias 209 -> 169 (3.5 TB/s), with
+// a bias per tile, 16 tiles, 148 -> 110 (4.9 TB/s), with a soft-cap 200 -> 169; 30
+// tiles 1001 x 1003 x 64, shared bias 69 -> 52, no bias 55 -> 42. A shared bias
+// with the tiles of an XCD one after another (the order of the other calls):
+// 182.
 constexpr int kRowBufBytes = 32 * 1024;   // one K block (128 rows x 16 CH bytes), or the epilogue staging
 
 template <int CH>
@@ -383,7 +397,7 @@ __device__ __forceinline__ int row_swz(int row) {
     return CH == 16 ? (row & 15) : CH == 8 ? ((row >> 1) & 7) : ((row >> 2) & 3);
 }
 
-template <typename T, int CH>
+template <typename T, int CH, int POST, bool VEC>
 __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs a, int64_t nqb, int64_t npieces,
                                                                     int tpw) {
 #pragma clang fp contract(off)
@@ -396,9 +410,14 @@ __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs 
     const int r = lane & 31, half = lane >> 5;
     const int64_t total = gridDim.x, n = blockIdx.x, per = total / 8;
     const int64_t id = n < 8 * per ? (n % 8) * per + n / 8 : n;
-    const int64_t piece = id % npieces;
-    const int64_t qb = (id / npieces) % nqb;
-    const int64_t bt = id / (npieces * nqb);
+    int64_t piece = id % npieces, qb = (id / npieces) % nqb, bt = id / (npieces * nqb);
+    if ((POST & QK_POST_BIAS) != 0 && a.bias_sb == 0 && (a.batch & 7) == 0) {
+        // A bias that all tiles share: an XCD's tiles (n mod 8 again) run side by
+        // side, so that its L2 serves a bias block to all of them
+        bt = n % a.batch;
+        piece = (n / a.batch) % npieces;
+        qb = n / (a.batch * npieces);
+    }
     const int64_t nkb = (a.N + kMfmaBlock - 1) / kMfmaBlock;
     const int64_t kb_begin = piece * tpw;
     const int64_t kb_end = min(nkb, kb_begin + tpw);
@@ -449,6 +468,34 @@ __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs 
         const int buf = (int)((kb - kb_begin) & 1);
         if (kb + 1 < kb_end) copy_k(kb + 1, buf ^ 1);
         qk_lds_u8* kl = lds + buf * kRowBufBytes;
+        const int64_t j0 = kb * kMfmaBlock + (wave & 1) * 64;
+        // Bias of rows 32 x .. +31 of the wavefront's block; rows and columns past
+        // the end repeat the last one. (The row and lane are hidden from the compiler,
+        // which would otherwise keep every row's address over the K blocks and spill.)
+        [[maybe_unused]] float bias[32];
+        auto load_bias = [&](int x) {
+            int ln = lane, row0 = (int)min(i0 + 32 * x, a.M - 1);
+            int left = (int)(a.M - 1 - row0);
+            asm volatile("" : "+v"(ln), "+s"(left));
+            const float* bb = a.bias + bt * a.bias_sb + row0 * a.bias_sm;
+            if constexpr (VEC) {
+                bb += min(j0 + 4 * (ln & 15), a.N - 4);
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const qk_f32x4 v = *(const qk_f32x4*)(bb + min(4 * it + (ln >> 4), left) * a.bias_sm);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) bias[4 * it + u] = v[u];
+                }
+            } else {
+                bb += min(j0 + ln, a.N - 1) * a.bias_sn;
+#pragma unroll
+                for (int it = 0; it < 32; ++it) {
+                    bias[it] = *bb;
+                    bb += it < left ? a.bias_sm : 0;
+                }
+            }
+        };
+        if constexpr ((POST & QK_POST_BIAS) != 0) load_bias(0);
         qk_f32x16 acc[2][2];
 #pragma unroll
         for (int x = 0; x < 2; ++x)
@@ -470,14 +517,23 @@ __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs 
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K block kb+1 has landed
         __syncthreads();                      // ... for every wavefront; buffer `kl` is free for staging
-        // epilogue as in qk_score_mfma_kernel, with 32-bit lane offsets from the wavefront's
-        // block (the launcher checks that 64 rows and 64 columns of strides fit)
-        const int64_t j0 = kb * kMfmaBlock + (wave & 1) * 64;
+        // Epilogue through a 32-row buffer of this wavefront (the block of K is no
+        // longer read), 32-bit lane offsets from the wavefront's block (the launcher
+        // checks that 64 rows and 64 columns of strides fit).
         qk_lds_u8* stg = kl + wave * 32 * 256;
-        const int col = 4 * (lane & 15);
-        const int64_t jb = j0 + col;
         float* cw = a.c + bt * a.c_sb + i0 * a.c_sm + j0 * a.c_sn;
-        const int csm = (int)a.c_sm, csn = (int)a.c_sn;
+        int csm = (int)a.c_sm;
+        const int csn = (int)a.c_sn;
+        if constexpr ((POST & QK_POST_BIAS) != 0) asm volatile("" : "+s"(csm));  // (as above)
+        auto post = [&](float v, float b) {
+#pragma clang fp contract(off)  // (a lambda's body does not take the function's pragma)
+            if (a.has_scale) v = v * a.scale;
+            if constexpr ((POST & QK_POST_BIAS) != 0) v = v + b;
+            if constexpr ((POST & QK_POST_CAP) != 0) v = a.softcap * tanhf(v / a.softcap);
+            return v;
+        };
+        // (with registers held for the bias every index into them must be constant)
+        constexpr bool BIASED = (POST & QK_POST_BIAS) != 0;
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -489,30 +545,50 @@ __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs 
                                  qk_f32x4{acc[x][y][4 * g], acc[x][y][4 * g + 1], acc[x][y][4 * g + 2],
                                           acc[x][y][4 * g + 3]});
                 }
-            __syncthreads();
-            // two rows of stores per unrolled step: more would hoist every row's address out of
-            // the K-block loop and leave too few registers for two wavefronts per SIMD
-#pragma unroll 2
-            for (int it = 0; it < 8; ++it) {
-                const int row = 4 * it + (lane >> 4);
-                const int rr = 32 * x + row;   // row in the wavefront's block
-                if (i0 + rr >= a.M || jb >= a.N) continue;
-                const qk_f32x4 raw = lds_read_f4(stg + row * 256 + 16 * ((lane & 15) ^ (row & 15)));
-                float v[4] = {raw[0], raw[1], raw[2], raw[3]};
+            // (the buffer is the wavefront's own and its LDS operations stay in order)
+            asm volatile("" ::: "memory");
+            if constexpr (VEC) {
+                const int col = 4 * (lane & 15);
+                auto rows4 = [&](int it) {
+                    const int row = 4 * it + (lane >> 4);
+                    const int rr = 32 * x + row;  // row in the wavefront's block
+                    if (i0 + rr >= a.M || j0 + col >= a.N) return;
+                    const qk_f32x4 raw = lds_read_f4(stg + row * 256 + 16 * ((lane & 15) ^ (row & 15)));
+                    qk_f32x4 v;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = a.has_scale ? v[u] * a.scale : v[u];
-                if (a.vec4 && jb + 3 < a.N) {
-                    *(float4*)(cw + (rr * csm + col)) = make_float4(v[0], v[1], v[2], v[3]);
+                    for (int u = 0; u < 4; ++u) v[u] = post(raw[u], BIASED ? bias[4 * it + u] : 0.0f);
+                    *(qk_f32x4*)(cw + (rr * csm + col)) = v;
+                };
+                // without a bias, two rows of stores per unrolled step: more would hoist every row's
+                // address out of the K-block loop and leave too few registers for two wavefronts per SIMD
+                if constexpr (BIASED) {
+#pragma unroll
+                    for (int it = 0; it < 8; ++it) rows4(it);
                 } else {
+#pragma unroll 2
+                    for (int it = 0; it < 8; ++it) rows4(it);
+                }
+            } else {
+                auto row1 = [&](int row) {
+                    const int rr = 32 * x + row;
+                    if (i0 + rr >= a.M || j0 + lane >= a.N) return;
+                    const float raw = *(const qk_lds_f32*)(stg + row * 256 + 16 * ((lane >> 2) ^ (row & 15)) + 4 * (lane & 3));
+                    cw[rr * csm + lane * csn] = post(raw, BIASED ? bias[row] : 0.0f);
+                };
+                if constexpr (BIASED) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        if (jb + u >= a.N) break;
-                        cw[rr * csm + (col + u) * csn] = v[u];
-                    }
+                    for (int row = 0; row < 32; ++row) row1(row);
+                } else {
+#pragma unroll 4
+                    for (int row = 0; row < 32; ++row) row1(row);
                 }
             }
-            __syncthreads();  // the next pass (or the next K block's copy) reuses the buffer
+            if constexpr (BIASED) {
+                if (x == 0) load_bias(1);
+            }
+            asm volatile("" ::: "memory");  // the next pass reuses the buffer
         }
+        __syncthreads();  // the next K block's copy reuses the buffers
     }
 }
 
@@ -525,6 +601,28 @@ inline int64_t rows_blocks_per_workgroup(int64_t tiles, int64_t nkb) {
     int64_t tpw = tiles / 4096;
     if (tpw < 4) tpw = std::min<int64_t>(4, std::max<int64_t>(1, tiles / 512));
     return std::min(tpw, nkb);
+}
+
+template <typename T, int CH, int POST>
+void launch_rows_post(const QkScoreArgs& x, bool vec, int64_t nqb, int64_t npieces, int tpw, hipStream_t s) {
+    const dim3 grid((unsigned)(x.batch * nqb * npieces));
+    if (vec) hipLaunchKernelGGL((qk_score_mfma_rows_kernel<T, CH, POST, true>), grid, dim3(256), 0, s, x, nqb, npieces, tpw);
+    else hipLaunchKernelGGL((qk_score_mfma_rows_kernel<T, CH, POST, false>), grid, dim3(256), 0, s, x, nqb, npieces, tpw);
+}
+template <typename T, int CH>
+void launch_rows_ch(const QkScoreArgs& x, bool vec, int64_t nqb, int64_t npieces, int tpw, hipStream_t s) {
+    const bool bias = x.bias != nullptr, cap = x.softcap > 0.0f;
+    if (bias && cap) launch_rows_post<T, CH, QK_POST_BIAS_CAP>(x, vec, nqb, npieces, tpw, s);
+    else if (bias) launch_rows_post<T, CH, QK_POST_BIAS>(x, vec, nqb, npieces, tpw, s);
+    else if (cap) launch_rows_post<T, CH, QK_POST_CAP>(x, vec, nqb, npieces, tpw, s);
+    else launch_rows_post<T, CH, QK_POST_NONE>(x, vec, nqb, npieces, tpw, s);
+}
+template <typename T>
+hipError_t launch_rows_k(const QkScoreArgs& x, bool vec, int64_t nqb, int64_t npieces, int tpw, hipStream_t s) {
+    if (x.K <= 32) launch_rows_ch<T, 4>(x, vec, nqb, npieces, tpw, s);
+    else if (x.K <= 64) launch_rows_ch<T, 8>(x, vec, nqb, npieces, tpw, s);
+    else launch_rows_ch<T, 16>(x, vec, nqb, npieces, tpw, s);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -543,36 +641,26 @@ hipError_t launch_qk_score_mfma(const QkScoreArgs& a, int dtype, hipStream_t s) 
     const bool c_vec = a.c_sn == 1 && a.c_sm % 4 == 0 && a.c_sb % 4 == 0 && al16(a.c);
     const bool b_vec = a.bias == nullptr ||
                        (a.bias_sn == 1 && a.bias_sm % 4 == 0 && a.bias_sb % 4 == 0 && al16(a.bias));
-    // Scores only (no bias, no soft-cap), K <= 128, lane offsets within 32 bits: the row kernel.
+    // K <= 128, lane offsets within 32 bits: the row kernel.
     const int64_t lim31 = int64_t(1) << 31;
-    const bool rows = a.bias == nullptr && !(a.softcap > 0.0f) && a.K <= 128 &&
-                      (kMfmaBlock - 1) * a.b_sn + a.K < lim31 && 63 * (a.c_sm + a.c_sn) + 4 < lim31 &&
-                      a.b_sn >= 0 && a.c_sm >= 0 && a.c_sn >= 0;
+    const bool rows = a.K <= 128 && (kMfmaBlock - 1) * a.b_sn + a.K < lim31 &&
+                      63 * (a.c_sm + a.c_sn) + 4 < lim31 && a.b_sn >= 0 && a.c_sm >= 0 && a.c_sn >= 0;
     if (rows) {
         const int64_t nqb = (a.M + kMfmaBlock - 1) / kMfmaBlock, nkb = (a.N + kMfmaBlock - 1) / kMfmaBlock;
         const int64_t max_grid = (int64_t(1) << 31) - 1;
+        const bool vec = c_vec && b_vec && a.N % 4 == 0;
         for (int64_t b0 = 0; b0 < a.batch;) {
             QkScoreArgs x = a;
-            x.vec4 = c_vec;
             x.batch = std::min<int64_t>(a.batch - b0, std::max<int64_t>(1, max_grid / (nqb * nkb)));
             x.q = (const char*)a.q + b0 * a.a_sb * 2;
             x.k = (const char*)a.k + b0 * a.b_sb * 2;
             x.c = a.c + b0 * a.c_sb;
+            if (a.bias != nullptr) x.bias = a.bias + b0 * a.bias_sb;
             const int64_t tiles = x.batch * nqb * nkb;
             const int64_t tpw = rows_blocks_per_workgroup(tiles, nkb);
             const int64_t npieces = (nkb + tpw - 1) / tpw;
-            const dim3 grid((unsigned)(x.batch * nqb * npieces));
-            const int K = (int)a.K;
-            if (dtype == DT_BF16) {
-                if (K <= 32) hipLaunchKernelGGL((qk_score_mfma_rows_kernel<__bf16, 4>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-                else if (K <= 64) hipLaunchKernelGGL((qk_score_mfma_rows_kernel<__bf16, 8>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-                else hipLaunchKernelGGL((qk_score_mfma_rows_kernel<__bf16, 16>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-            } else {
-                if (K <= 32) hipLaunchKernelGGL((qk_score_mfma_rows_kernel<_Float16, 4>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-                else if (K <= 64) hipLaunchKernelGGL((qk_score_mfma_rows_kernel<_Float16, 8>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-                else hipLaunchKernelGGL((qk_score_mfma_rows_kernel<_Float16, 16>), grid, dim3(256), 0, s, x, nqb, npieces, (int)tpw);
-            }
-            const hipError_t e = hipGetLastError();
+            const hipError_t e = dtype == DT_BF16 ? launch_rows_k<__bf16>(x, vec, nqb, npieces, (int)tpw, s)
+                                                  : launch_rows_k<_Float16>(x, vec, nqb, npieces, (int)tpw, s);
             if (e != hipSuccess) return e;
             b0 += x.batch;
         }

@@ -92,6 +92,36 @@ def test_exact_kernel_bit_exact(ofh, dt, shape):
         np.testing.assert_array_equal(_bits(got.cpu().numpy()), _bits(want))
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("T,M,N,K", [(8, 129, 132, 64), (3, 64, 63, 32), (16, 200, 260, 128), (1, 1, 1, 8),
+                                     (5, 257, 129, 72), (2, 33, 600, 16)])
+def test_mfma_post_ops_at_block_edges(ofh, dt, T, M, N, K):
+    """The row kernel's bias (shared, with the order of workgroups that goes with
+    it from 8 tiles up, and per tile), soft-cap and both, with rows of 16-byte
+    alignment and without, past its row and column edges; nothing is written
+    outside the scores. The bound is the sum's, plus the roundings after it: the
+    soft-cap has slope at most 1, and tanhf a few units in the last place."""
+    rng = np.random.default_rng(T + N)
+    tq, uq = to_device(rng.standard_normal((T, M, K), dtype=np.float32), dt)
+    tk, uk = to_device(rng.standard_normal((T, N, K), dtype=np.float32), dt)
+    shared = rng.standard_normal((M, N), dtype=np.float32)
+    for bias in (None, shared, rng.standard_normal((T, M, N), dtype=np.float32)):
+        for cap in (0.0, 3.0):
+            want = O.qk_score_tile(uq, uk, scale=0.125, bias=bias)
+            bound = _mfma_bound(uq, uk, 0.125, want)
+            if cap > 0:
+                want = cap * np.tanh(want.astype(np.float64) / cap)
+                bound = bound + 8 * 2.0 ** -24 * cap
+            for pad in (0, 1):
+                out = torch.full((T, M + 1, N + pad), 7.0, device="cuda")
+                _run(ofh, tq, tk, scale=0.125, bias=None if bias is None else _dev32(bias), softcap=cap,
+                     out=out[:, :M, :N], algorithm=ofh.QK_MFMA)
+                host = out.cpu().numpy()
+                assert (np.abs(host[:, :M, :N] - want) <= bound).all()
+                host[:, :M, :N] = 7.0
+                assert (host == 7.0).all()
+
+
 @pytest.mark.parametrize("dt", ["f32", "f16"])
 @pytest.mark.parametrize("T,M,N,K", [(200, 65, 129, 33), (1100, 63, 40, 5), (3, 65, 129, 33), (2, 31, 33, 31)])
 def test_exact_kernel_block_edges(ofh, dt, T, M, N, K):
