@@ -79,6 +79,25 @@ class AttentionParams(ctypes.Structure):
     ]
 
 
+def _flat_fields(fields):
+    """The fields with their arrays taken apart: the same layout, for one positional
+    construction instead of an assignment per field and array element."""
+    flat = []
+    for name, t in fields:
+        if isinstance(t, type) and issubclass(t, ctypes.Array):
+            flat += [(f"{name}{i}", t._type_) for i in range(t._length_)]
+        else:
+            flat.append((name, t))
+    return flat
+
+
+class _FlatAttentionParams(ctypes.Structure):
+    _fields_ = _flat_fields(AttentionParams._fields_)
+
+
+assert ctypes.sizeof(_FlatAttentionParams) == ctypes.sizeof(AttentionParams)
+
+
 class LaunchInfo(ctypes.Structure):
     _fields_ = [
         ("algorithm", ctypes.c_int32),
@@ -168,6 +187,11 @@ def lib() -> ctypes.CDLL:
                    "ofh_attention_fwd_host",
                    "ofh_attention_launch_info", "ofh_attention_useful_flops"):
             getattr(L, fn).restype = ctypes.c_int
+        # attention_fwd's own handle of the entry (its parameters are built flat)
+        fwd = L["ofh_attention_fwd"]
+        fwd.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_size_t, ctypes.c_void_p]
+        fwd.restype = ctypes.c_int
+        L.fwd_flat = fwd
         _lib = L
     return _lib
 
@@ -240,14 +264,43 @@ def workspace_bytes(p: AttentionParams) -> int:
 # ---------------------------------------------------------------------------
 # torch-facing helpers (device tensors)
 
+_torch_module = None
+_DTYPE_CODES: dict = {}
+
+
 def _torch():
-    import torch  # noqa: PLC0415
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch  # noqa: PLC0415
+        _DTYPE_CODES.update({torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16})
+        _torch_module = torch
+    return _torch_module
 
 
 def dtype_code(t) -> int:
-    torch = _torch()
-    return {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16}[t]
+    _torch()
+    return _DTYPE_CODES[t]
+
+
+def _raw_stream(torch, device) -> int:
+    """The current stream's handle on a GPU device."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def _plain_inputs_fit(torch, q, k, v) -> bool:
+    """What _check_attention_inputs asks of q, k and v, in one pass: true only where
+    it would find nothing to report about them."""
+    tensor = torch.Tensor
+    if not (isinstance(q, tensor) and isinstance(k, tensor) and isinstance(v, tensor)):
+        return False
+    qs, ks, vs, dt, dev = q.shape, k.shape, v.shape, q.dtype, q.device
+    if not (len(qs) == 4 and len(ks) == 4 and len(vs) == 4 and dt in _DTYPE_CODES and k.dtype == dt and v.dtype == dt):
+        return False
+    a, b, c = q.stride(), k.stride(), v.stride()
+    return (a[3] == 1 and b[3] == 1 and c[3] == 1 and min(a) >= 0 and min(b) >= 0 and min(c) >= 0
+            and ks[0] == qs[0] and ks[1] == qs[1] and vs[0] == qs[0] and vs[1] == qs[1]
+            and ks[3] == qs[3] and vs[2] == ks[2] and dev.type == "cuda" and k.device == dev and v.device == dev)
 
 
 def _check_attention_inputs(q, k, v, mask, mask_block_size, alibi_slopes, bias, out, out_dtype,
@@ -336,37 +389,39 @@ def attention_fwd(q, k, v, *, scale: float | None = None, causal: bool = False, 
     f32 device [H]. bias: f32 device [M,N] (shared) or [B,H,M,N]. Returns out.
     Raises ValueError before any launch when the arguments do not fit together."""
     torch = _torch()
-    _check_attention_inputs(q, k, v, mask, mask_block_size, alibi_slopes, bias, out, out_dtype,
-                            workspace)
+    # (with q, k and v alone there is nothing else to check)
+    alone = (mask is None and alibi_slopes is None and bias is None and out is None and out_dtype is None
+             and workspace is None)
+    if not (alone and _plain_inputs_fit(torch, q, k, v)):
+        _check_attention_inputs(q, k, v, mask, mask_block_size, alibi_slopes, bias, out, out_dtype,
+                                workspace)
     B, H, M, D = q.shape
     N, Dv = k.shape[2], v.shape[3]
     if out is None:
         out = torch.empty((B, H, M, Dv), device=q.device,
                           dtype=q.dtype if out_dtype is None else out_dtype)
-    kw = {}
+    mask_args = (None, 0, 0, 0, 0)
     if mask is not None:
-        kw.update(mask_allowed=mask.data_ptr(), mask_query_block_size=int(mask_block_size[0]),
-                  mask_key_block_size=int(mask_block_size[1]), mask_query_blocks=mask.shape[0],
-                  mask_key_blocks=mask.shape[1])
-    bias_kind = BIAS_NONE
+        mask_args = (mask.data_ptr(), int(mask_block_size[0]), int(mask_block_size[1]), mask.shape[0], mask.shape[1])
+    bias_kind, slopes_ptr, bias_ptr, bias_strides = BIAS_NONE, None, None, (0, 0, 0)
     if alibi_slopes is not None:
-        bias_kind = BIAS_ALIBI
-        kw["alibi_slopes"] = alibi_slopes.data_ptr()
+        bias_kind, slopes_ptr = BIAS_ALIBI, alibi_slopes.data_ptr()
     elif bias is not None:
-        bias_kind = BIAS_DENSE
-        kw["bias"] = bias.data_ptr()
+        bias_kind, bias_ptr = BIAS_DENSE, bias.data_ptr()
         if bias.dim() == 4:
-            kw["bias_strides"] = (bias.stride(0), bias.stride(1), bias.stride(2))
-    p = make_params(B, H, M, N, D, Dv, dtype=dtype_code(q.dtype), out_dtype=dtype_code(out.dtype),
-                    scale=(1.0 / math.sqrt(D)) if scale is None else scale, causal=causal,
-                    bias_kind=bias_kind, softcap=softcap, algorithm=algorithm,
-                    strides=[(t.stride(0), t.stride(1), t.stride(2)) for t in (q, k, v, out)],
-                    max_key_splits=max_key_splits, **kw)
+            bias_strides = bias.stride()[:3]
+    p = _FlatAttentionParams(
+        ctypes.sizeof(AttentionParams), B, H, M, N, D, Dv, _DTYPE_CODES[q.dtype], _DTYPE_CODES[out.dtype],
+        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3],
+        (1.0 / math.sqrt(D)) if scale is None else scale, int(bool(causal)), *mask_args, bias_kind, slopes_ptr,
+        bias_ptr, *bias_strides, softcap, algorithm, max_key_splits)
     if stream is None:
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+        stream = _raw_stream(torch, q.device)
     ws_ptr, ws_bytes = (0, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
-    check(lib().ofh_attention_fwd(ctypes.byref(p), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                  out.data_ptr(), ws_ptr or None, ws_bytes, stream))
+    rc = lib().fwd_flat(ctypes.addressof(p), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws_ptr or None,
+                        ws_bytes, stream)
+    if rc != OFH_SUCCESS:
+        check(rc)
     return out
 
 
@@ -404,7 +459,7 @@ def qk_score_tile(q, k, *, scale: float | None = None, bias=None, softcap: float
     p.softcap = softcap
     p.algorithm = algorithm
     if stream is None:
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+        stream = _raw_stream(torch, q.device)
     check(lib().ofh_qk_score_tile(ctypes.byref(p), q.data_ptr(), k.data_ptr(), out.data_ptr(),
                                   stream))
     return out

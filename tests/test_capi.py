@@ -412,6 +412,20 @@ def test_key_group_choice(ofh):
         assert "keygroups" not in other, other
 
 
+def test_flat_params_layout(ofh):
+    """attention_fwd's positionally built parameters are byte for byte the
+    ofh_attention_params that make_params fills."""
+    F = ofh
+    values = dict(dtype=1, out_dtype=0, scale=0.25, causal=True, mask_allowed=11, mask_query_block_size=12,
+                  mask_key_block_size=13, mask_query_blocks=14, mask_key_blocks=15, bias_kind=2, alibi_slopes=16,
+                  bias=17, bias_strides=(18, 19, 20), softcap=2.5, algorithm=1, max_key_splits=3,
+                  strides=[(1, 2, 3), (4, 5, 6), (7, 8, 9), (10, 11, 12)])
+    p = F.make_params(2, 3, 4, 5, 6, 7, **values)
+    flat = F._FlatAttentionParams(ctypes.sizeof(F.AttentionParams), 2, 3, 4, 5, 6, 7, 1, 0, *range(1, 13), 0.25, 1,
+                                  11, 12, 13, 14, 15, 2, 16, 17, 18, 19, 20, 2.5, 1, 3)
+    assert bytes(p) == bytes(flat)
+
+
 def test_useful_flops_match_workloads(ofh):
     import onednn_flash_configs as C
     F = ofh
