@@ -51,6 +51,7 @@ struct Resolved {
     bool pair_split;     // causal: query tile pairs, each tile split in key_splits ranges of its own length
     int groups;          // > 0: wavefront groups split the keys inside a workgroup (flash_fwd_keygroups_kernel)
     bool staged_bias;    // 16-bit dense bias copied through LDS (flash_fwd_bias_kernel)
+    bool f32_waves;      // fp32: 32-row blocks of eight wavefronts (flash_fwd_f32_waves_kernel)
     bool decode;         // a few query rows: flash_fwd_decode_kernel, one workgroup per head and key split
     int kdim;            // head dim of the MFMA kernel: max(D, Dv) rounded up to a multiple of 32
 };
@@ -337,6 +338,53 @@ void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
     r.num_k_tiles = (int)((N + r.block_n - 1) / r.block_n);
 }
 
+// fp32 calls with more than half a 32-row block per CU: eight wavefronts per
+// block instead of the key split of 32-row blocks or the 128-row tiles, whose
+// partial rounds and merge they avoid. Up to 128 blocks the split keeps more
+// CUs busy, and 16-row blocks cost half (D64 H8 N512 9.7 us against 14.0).
+// Measured, split or tiles against eight wavefronts (us): D64 H16 N512 32.2 /
+// 14.5, H8 N1000 47.7 / 25.0, H64 N384 54.4 / 31.4, H16 N1536 133 / 99, causal
+// H16 N1000 51.0 / 29.8, H32 N1536 177 / 117; D128 H16 N256 25.1 / 14.8, H8
+// N1000 66.1 / 46.5, causal H64 N1000 320 / 214. With every CU busy for several
+// rounds the tiles, which share each K/V tile among more rows, win: D64 H64
+// N1000 155 / 184, H8 N4096 318 / 331, D128 H32 N1000 162 / 178; long causal
+// calls gain little or nothing (paired tiles: D64 H16 N2048 104 / 97, H8 N4096
+// 175 / 176) and keep their plans, as do 96-wide ones, which this kernel
+// multiplies as 128 (H16 N2048 243 / 336). A partly filled last round costs a
+// whole one (D64 H17 N1069, 578 blocks: 66 / 75), causal blocks in one round
+// wait for the longest (D128 H5 N826, 130 blocks: 37 / 38), and with fewer than
+// eight key tiles wavefronts stand idle (D128 H128 N183 37 / 41; causal rows far
+// past the last key see all of few keys: D128 H17 M3043 N281 112 / 124). Causal
+// pairs with a key split over more than 1024 keys keep that plan, on whose
+// workspace and launch description their callers may rely. So do more than three
+// rounds of fewer than 256 rows per head (D64 H128 M221 N1094 102 / 101).
+void choose_f32_waves(const ofh_attention_params* p, Resolved& r) {
+    if (p->dtype != OFH_DTYPE_F32 || p->max_key_splits != 0 || r.decode || r.general_mod || r.tile_list ||
+        r.block_m == ofh::kRowsF32Narrow || (r.kdim != 64 && r.kdim != 128))
+        return;
+    const int64_t M = (int64_t)p->query_tokens, N = (int64_t)p->key_tokens;
+    const int64_t tiles = (M + ofh::kRowsF32 - 1) / ofh::kRowsF32, blocks = (int64_t)p->batch * p->heads * tiles;
+    const int64_t rounds = (blocks + kComputeUnits - 1) / kComputeUnits;
+    const int64_t keys = p->causal ? std::min(M, N) : N;
+    if (2 * blocks <= kComputeUnits || keys < 128 || (r.pair_split && N > 1024)) return;
+    if (rounds == 1 ? (p->causal ? 4 * blocks < 3 * kComputeUnits || N > 2048 : N > 4096)
+        : N < 256 || (rounds > 3 && M < 256) ? true
+        : p->causal ? rounds > 8 || 2 * N < M || N > (r.kdim == 64 ? 1536 : 2048)
+                    : rounds > (r.kdim == 64 ? 4 : 3) || N > 1536 ||
+                          8 * blocks < (N <= 512 ? 6 : 7) * kComputeUnits * rounds)
+        return;
+    r.f32_waves = true;
+    r.key_splits = 1;
+    r.split_tiles = 1 << 30;
+    r.pair_split = false;
+    r.paired = false;
+    r.block_m = ofh::kRowsF32;
+    r.block_n = 32;
+    r.threads = ofh::kF32WavesThreads;
+    r.num_q_tiles = (int)tiles;
+    r.num_k_tiles = (int)((N + r.block_n - 1) / r.block_n);
+}
+
 int resolve(const ofh_attention_params* p, const void* q, const void* k, const void* v,
             const void* out, Resolved& r) {
     contiguous_strides(r.qs, p->q_strides, p->heads, p->query_tokens, p->head_dim);
@@ -345,6 +393,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     contiguous_strides(r.os, p->o_strides, p->heads, p->query_tokens, p->value_dim);
     r.general_mod = p->bias_kind != OFH_BIAS_NONE || p->softcap > 0.0f;
     r.decode = false;
+    r.f32_waves = false;
     r.groups = 0;
     r.staged_bias = false;
 
@@ -465,6 +514,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
         return set_error(OFH_ERROR_UNSUPPORTED, "block-mask tile list entry cannot encode this tiling");
     choose_key_splits(p, r);
     choose_key_groups(p, r);
+    choose_f32_waves(p, r);
     set_lds_list(p, r);
     return OFH_SUCCESS;
 }
@@ -793,6 +843,7 @@ int fwd_impl(const ofh_attention_params* p, const void* q, const void* k, const 
     }
     OFH_HIP_CHECK(r.staged_bias ? ofh::launch_bias(a, p->dtype, stream)
                   : r.groups ? ofh::launch_key_groups(a, p->dtype, r.groups, stream)
+                  : r.f32_waves ? ofh::launch_f32_waves(a, stream)
                   : r.decode ? ofh::launch_decode(a, p->dtype, stream)
                              : ofh::launch_flash_mfma(a, p->dtype, r.general_mod, stream));
     if (r.key_splits > 1 && a.split_counters == nullptr)
@@ -1025,6 +1076,9 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
         info->key_splits = r.key_splits;
         info->merge_in_launch = merge_in_launch(p, r) ? 1 : 0;
         name = r.decode ? decode_kernel_name(p->dtype, (int)p->head_dim, (int)p->value_dim)
+               : r.f32_waves
+                   ? (p->head_dim <= 64 && p->value_dim <= 64 ? "flash_fwd_f32_waves_kernel<64>"
+                                                              : "flash_fwd_f32_waves_kernel<128>")
                : (p->dtype == OFH_DTYPE_F32 && (r.block_m == ofh::kRowsF32 || r.block_m == ofh::kRowsF32Narrow))
                    ? rows32_kernel_name(r.kdim, r.general_mod, r.block_m == ofh::kRowsF32Narrow)
                    : ofh::flash_mfma_kernel_name(p->dtype, r.kdim, r.general_mod, r.tile_list, r.threads);

@@ -186,6 +186,10 @@ hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipS
 hipError_t launch_key_groups(const FwdArgs& a, int dtype, int groups, hipStream_t s);
 // Keys of a staged tile: what one step of all groups covers.
 int key_group_keys(int kernel_dim, int groups);
+// fp32 calls on 32-row blocks of eight wavefronts (flash_f32_waves.hip): plain
+// scale, no block mask, head dims up to 128, no key split.
+constexpr int kF32WavesThreads = 512;
+hipError_t launch_f32_waves(const FwdArgs& a, hipStream_t s);
 // 16-bit calls with a dense bias and no block mask, kernel head dims up to 128
 // (flash_bias.hip), on the score_mod kernel's tiling and plans, where the bias
 // can be copied 16 bytes at a time: aligned rows of whole chunks, and 32-bit

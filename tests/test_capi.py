@@ -412,6 +412,27 @@ def test_key_group_choice(ofh):
         assert "keygroups" not in other, other
 
 
+def test_f32_waves_choice(ofh):
+    """Eight-wavefront blocks take plain fp32 calls with more than half a
+    32-row block per CU and few rounds; every other call keeps its plan."""
+    F = ofh
+
+    def name(B, H, M, N, D, **kw):
+        return F.launch_info(F.make_params(B, H, M, N, D, **kw)).kernel_name.decode()
+
+    for call in [(1, 16, 512, 512, 64), (1, 64, 384, 384, 64), (3, 8, 256, 256, 128), (1, 8, 1000, 1000, 100)]:
+        for causal in [False, True]:
+            width = 64 if call[4] <= 64 else 128
+            assert name(*call, causal=causal) == f"flash_fwd_f32_waves_kernel<{width}>"
+            for kw in [dict(max_key_splits=1), dict(softcap=5.0), dict(dtype=F.DTYPE_BF16)]:
+                assert "waves" not in name(*call, causal=causal, **kw)
+    for other in [name(1, 8, 512, 512, 64), name(1, 64, 1000, 1000, 64), name(1, 16, 1000, 1000, 32),
+                  name(1, 17, 512, 512, 64), name(1, 8, 1000, 1000, 96), name(2, 8, 2048, 2048, 64, causal=True),
+                  name(1, 64, 256, 100, 64), name(1, 64, 64, 1000, 128, causal=True),
+                  name(1, 16, 1000, 1000, 160), name(1, 16, 2048, 2048, 96, causal=True)]:
+        assert "waves" not in other, other
+
+
 def test_flat_params_layout(ofh):
     """attention_fwd's positionally built parameters are byte for byte the
     ofh_attention_params that make_params fills."""
