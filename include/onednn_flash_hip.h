@@ -67,8 +67,11 @@ typedef enum ofh_bias_kind {
  * is supported (head_dim and value_dim multiples of 4 for fp32 and of 8 for
  * bf16/fp16, up to 256, D != Dv allowed: the kernel of max(D, Dv)
  * rounded up to 32 runs with the padding zeroed in place; 16-byte aligned
- * rows) and the rowwise kernel otherwise. ROWWISE is the exact two-pass
- * softmax of standard_attention, run on the GPU one query row per wavefront. */
+ * rows) and the rowwise kernel otherwise; of those shapes, a few query rows
+ * against many keys (decoding: no mask, bias, soft-cap or causal rule) run on
+ * a vector kernel. ROWWISE is the exact two-pass softmax of
+ * standard_attention, run on the GPU in 32-row blocks up to head_dim and
+ * value_dim 256 and one query row per wavefront above. */
 typedef enum ofh_algorithm {
     OFH_ALGO_AUTO = 0,
     OFH_ALGO_FLASH_MFMA = 1,
