@@ -344,7 +344,7 @@ void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
 // CUs busy, and 16-row blocks cost half (D64 H8 N512 9.7 us against 14.0).
 // Measured, split or tiles against eight wavefronts (us): D64 H16 N512 32.2 /
 // 14.5, H8 N1000 47.7 / 25.0, H64 N384 54.4 / 31.4, H16 N1536 133 / 99, causal
-// H16 N1000 51.0 / 29.8, H32 N1536 177 / 117; D128 H16 N256 25.1 / 14.8, H8
+// H16 N1000 51.0 / 29.8, H32 N768 62.1 / 37.4; D128 H16 N256 25.1 / 14.8, H8
 // N1000 66.1 / 46.5, causal H64 N1000 320 / 214. With every CU busy for several
 // rounds the tiles, which share each K/V tile among more rows, win: D64 H64
 // N1000 155 / 184, H8 N4096 318 / 331, D128 H32 N1000 162 / 178; long causal

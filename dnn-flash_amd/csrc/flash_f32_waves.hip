@@ -12,7 +12,7 @@
 // Every wavefront keeps an online softmax state; the eight are folded in LDS.
 // One block per CU (80 to 88 KB of LDS), two wavefronts per SIMD: H8 N1000 D64
 // 47.7 -> 25.0 us (43 -> 82 TF of the 154 a large product reaches), causal
-// H32 N1536 D64 177 -> 117, H8 N1000 D128 66.1 -> 46.5.
+// H32 N768 D64 62.1 -> 37.4, H8 N1000 D128 66.1 -> 46.5.
 
 #include "flash_wave32.h"
 #include "ofh_kernels.h"
