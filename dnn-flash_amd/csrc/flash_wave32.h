@@ -462,7 +462,7 @@ struct Wave32 {
     // takes one chunk of 16 rows, 256 bytes apart. Rows past M and keys past N
     // repeat the last one (their scores are masked or never stored). Eight copies
     // of four rows each; rows are 16-byte aligned, N is a multiple of 4 and the
-    // row stride at most 2^24 (bias_can_be_staged).
+    // row stride within [0, 2^24] (bias_can_be_staged).
     static constexpr int BIAS_BYTES = 32 * BN * 4;  // per wavefront
     __device__ __forceinline__ void copy_bias(int e) {
         static_assert(BN == 64, "a bias row is 16 chunks");

@@ -192,10 +192,12 @@ constexpr int kF32WavesThreads = 512;
 hipError_t launch_f32_waves(const FwdArgs& a, hipStream_t s);
 // 16-bit calls with a dense bias and no block mask, kernel head dims up to 128
 // (flash_bias.hip), on the score_mod kernel's tiling and plans, where the bias
-// can be copied 16 bytes at a time: aligned rows of whole chunks, and 32-bit
-// offsets within 32 rows.
+// can be copied 16 bytes at a time: aligned rows of whole chunks, and offsets
+// within 32 rows that fit 32 bits without a sign (the copies add them to a
+// wavefront-uniform base, zero-extended). Rows that run backwards or lie
+// farther apart stay on the score_mod kernel, whose row pointers are 64-bit.
 inline bool bias_can_be_staged(const float* bias, int64_t N, int64_t sb, int64_t sh, int64_t sm) {
-    return ((uintptr_t)bias & 15) == 0 && ((N | sb | sh | sm) & 3) == 0 && sm <= (1 << 24);
+    return ((uintptr_t)bias & 15) == 0 && ((N | sb | sh | sm) & 3) == 0 && sm >= 0 && sm <= (1 << 24);
 }
 hipError_t launch_bias(const FwdArgs& a, int dtype, hipStream_t s);
 // Calls with a few query rows (decode_fwd.hip): plain scale, no mask.

@@ -412,6 +412,24 @@ def test_key_group_choice(ofh):
         assert "keygroups" not in other, other
 
 
+def test_staged_bias_choice(ofh):
+    """The dense-bias kernel copies rows at unsigned 32-bit offsets: bias rows that
+    run backwards or lie more than 2^24 elements apart stay on the score_mod
+    kernel. Batch and head strides are 64-bit there and may have any sign."""
+    F = ofh
+
+    def staged(*strides, bias=16):
+        p = F.make_params(2, 16, 2048, 2048, 64, dtype=F.DTYPE_F16, bias_kind=F.BIAS_DENSE, bias=bias)
+        p.bias_strides[:] = strides
+        return F.launch_info(p).kernel_name.decode().startswith("flash_fwd_bias_kernel<")
+
+    for sm in [0, 2048, 1 << 24]:
+        assert staged(4, -8, sm), sm
+    for sm in [-4, -2048, -(1 << 24), -(1 << 33), (1 << 24) + 4, 1 << 33, 2050]:
+        assert not staged(4, -8, sm), sm
+    assert not staged(0, 0, 2048, bias=24) and not staged(0, 2, 2048)
+
+
 def test_f32_waves_choice(ofh):
     """Eight-wavefront blocks take plain fp32 calls with more than half a
     32-row block per CU and few rounds; every other call keeps its plan."""

@@ -5,6 +5,8 @@ the same rounded inputs."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -58,3 +60,21 @@ def test_dense_bias_edges(ofh, dt, D, causal, splits):
                               max_key_splits=splits)
         ref = oracle_full(host, causal=causal, bias=bias.clip(min=-50), softcap=20.0)
         assert_bars(norm_error(cap.cpu().numpy(), ref)[0], dt, f"{dt} D{D} M{M} N{N} causal={causal} soft-cap")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_bias_rows_in_reverse(ofh, D):
+    """The C entry takes bias strides of either sign: rows stored last to first."""
+    F = ofh
+    M, N = 300, 260
+    dev, host = make_inputs("f16", 1, 3, M, N, D, seed=D)
+    bias = O.normal(77, (M, N), std=2.0)
+    t = torch.from_numpy(bias[::-1].copy()).cuda()
+    out = torch.empty(1, 3, M, D, device="cuda")
+    p = F.make_params(1, 3, M, N, D, dtype=F.DTYPE_F16, out_dtype=F.DTYPE_F32, scale=D ** -0.5,
+                      bias_kind=F.BIAS_DENSE, bias=t.data_ptr() + 4 * (M - 1) * N)
+    p.bias_strides[:] = (0, 0, -N)
+    assert F.launch_info(p).kernel_name.decode().startswith("flash_fwd_lockstep_kernel<f16,")
+    F.check(F.lib().ofh_attention_fwd(ctypes.byref(p), dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(),
+                                      out.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream))
+    assert_bars(norm_error(out.cpu().numpy(), oracle_full(host, bias=bias))[0], "f16", f"D{D} reversed bias rows")
