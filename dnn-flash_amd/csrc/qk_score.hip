@@ -13,6 +13,7 @@
 // summation order differs from the sequential sum (error within k * 2^-24 *
 // sum_k |q k| per score). It needs rows contiguous along k and 16-byte aligned.
 
+#include "k_chunks.h"
 #include "ofh_kernels.h"
 
 #include <algorithm>
@@ -79,15 +80,15 @@ __global__ __launch_bounds__(256) void qk_score_kernel(QkScoreArgs a) {
     Side sq = side((const T*)a.q + bt * a.a_sb, a.a_sm, a.a_sk, i0, a.M);
     Side sk = side((const T*)a.k + bt * a.b_sb, a.b_sn, a.b_sk, j0, a.N);
     float rq[LOADS], rk[LOADS];
-    auto load = [&](Side& d, float (&r)[LOADS], int kleft) {  // kleft: k elements from this chunk on
+    auto load = [&](Side& d, float (&r)[LOADS], int klen) {  // klen: k elements of this chunk
         const T* p = d.p;
-        if (d.rows == BT && kleft >= BK) {
+        if (d.rows == BT && klen == BK) {
 #pragma unroll
             for (int u = 0; u < LOADS; ++u) r[u] = to_f32(p[u * d.step]);
         } else {
 #pragma unroll
             for (int u = 0; u < LOADS; ++u)
-                r[u] = d.r0 + u * d.rs < d.rows && d.kk0 + u * d.kks < kleft ? to_f32(p[u * d.step]) : 0.0f;
+                r[u] = d.r0 + u * d.rs < d.rows && d.kk0 + u * d.kks < klen ? to_f32(p[u * d.step]) : 0.0f;
         }
         d.p += d.chunk;
     };
@@ -100,18 +101,20 @@ __global__ __launch_bounds__(256) void qk_score_kernel(QkScoreArgs a) {
     for (int x = 0; x < PT; ++x)
 #pragma unroll
         for (int y = 0; y < PT; ++y) acc[x][y] = 0.0f;
-    const int K = (int)a.K;
-    load(sq, rq, K);
-    load(sk, rk, K);
+    KChunks<BK> kc(a.K);
+    load(sq, rq, kc.len());
+    load(sk, rk, kc.len());
     put(sq, rq, qs[0]);
     put(sk, rk, ks[0]);
     __syncthreads();
     int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        const bool more = K - k0 > BK;
+    for (; kc.any(); kc.next()) {
+        const bool more = kc.more();
         if (more) {
-            load(sq, rq, K - k0 - BK);
-            load(sk, rk, K - k0 - BK);
+            KChunks<BK> nc = kc;
+            nc.next();
+            load(sq, rq, nc.len());
+            load(sk, rk, nc.len());
         }
         const float *ql = &qs[buf][GW * ty], *kl = &ks[buf][GW * tx];
         auto step = [&](int t) {
@@ -127,11 +130,12 @@ __global__ __launch_bounds__(256) void qk_score_kernel(QkScoreArgs a) {
 #pragma unroll
                 for (int y = 0; y < PT; ++y) acc[x][y] = acc[x][y] + qv[x / GW][x % GW] * kv[y / GW][y % GW];
         };
-        if (K - k0 >= BK) {
+        const int len = kc.len();
+        if (len == BK) {
 #pragma unroll 8
             for (int t = 0; t < BK; ++t) step(t);
         } else {
-            for (int t = 0; t < K - k0; ++t) step(t);
+            for (int t = 0; t < len; ++t) step(t);
         }
         if (more) {
             put(sq, rq, qs[buf ^ 1]);

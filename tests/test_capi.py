@@ -585,3 +585,14 @@ def test_stream_keys_of_library_scratch(tmp_path):
                     str(ROOT / "tests" / "cpp" / "stream_key_check.cpp"), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
+
+
+def test_score_tile_k_chunks(tmp_path):
+    """The exact score kernel's walk along k (csrc/k_chunks.h) covers k once, also
+    past 2^31, which the entry accepts. Built and run on the CPU."""
+    exe = tmp_path / "k_chunks_check"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'dnn-flash_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "cpp" / "k_chunks_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
