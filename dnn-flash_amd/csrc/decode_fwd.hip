@@ -1,5 +1,5 @@
 // Attention forward for calls with a few query rows against many keys
-// (decoding): up to kDecodeMaxRows rows of every head, plain scale, no mask.
+// (decoding): up to decode_max_rows() rows of every head, plain scale, no mask.
 //
 // What bounds it: reading K and V once. The matrix-core kernels give a
 // workgroup 32 to 256 query rows and stage K and V through LDS, so on such
@@ -132,15 +132,17 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void flash_fwd_decode_kernel(Fwd
     const int ks = (int)(split * range);
     const int ke = (int)min((int64_t)a.N, ks + range);
 
-    // Chunks at or past the row's real width repeat its last chunk: they meet
-    // zero query elements (K) or fill columns that are never stored (V).
+    // Lanes at or past the row's real width repeat its last chunk. Their K must not
+    // reach the score (an infinity there would be counted twice, as NaN against a
+    // zero query), V fills columns that are never stored.
+    const bool in_row = C::N * c < a.D;
     const T* Kp = (const T*)a.k + b * a.k_sb + h * a.k_sh + C::N * min(c, a.D / C::N - 1);
     const T* Vp = (const T*)a.v + b * a.v_sb + h * a.v_sh + C::N * min(c, a.Dv / C::N - 1);
     u32x4 q[MQ];
 #pragma unroll
     for (int i = 0; i < MQ; ++i) {
         q[i] = u32x4{0u, 0u, 0u, 0u};
-        if (C::N * c < a.D)
+        if (in_row)
             q[i] = *(const u32x4*)((const T*)a.q + b * a.q_sb + h * a.q_sh + (int64_t)min(i, a.M - 1) * a.q_sm + C::N * c);
     }
     float m[MQ], l[MQ], o[MQ][C::N];
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void flash_fwd_decode_kernel(Fwd
             float mx = m[i];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                s[u] = row_sum<LPR>(C::dot(kc[u], q[i])) * a.scale_log2;
+                s[u] = row_sum<LPR>(in_row ? C::dot(kc[u], q[i]) : 0.0f) * a.scale_log2;
                 if (!whole && k0 + u * RPI + sub >= ke) s[u] = kNegInf;
                 mx = fmaxf(mx, s[u]);
             }

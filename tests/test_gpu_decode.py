@@ -73,3 +73,20 @@ def test_decode_infinite_value_in_the_last_key(ofh, splits):
     assert out[0, 0, 0, 5] == np.inf
     out[0, 0, 0, 5] = 0
     assert np.isfinite(out).all()
+
+
+@pytest.mark.parametrize("dt,D", [("f32", 8), ("f32", 80), ("f32", 100), ("f32", 160), ("bf16", 32), ("f16", 96), ("bf16", 72)])
+@pytest.mark.parametrize("splits", [1, 0])
+def test_decode_infinite_key(ofh, dt, D, splits):
+    """Keys whose score is -inf through an infinity in the last chunk of their
+    row take weight 0, also where lanes past the row's width repeat that chunk."""
+    F = ofh
+    M = 3 if dt == "f32" else 2
+    dev, host = make_inputs(dt, 1, 2, M, 700, D, seed=D)
+    for q, k in [(dev[0], dev[1]), (host[0], host[1])]:
+        q[..., D - 2:] = 1.5
+        k[0, :, 3::7, D - 1] = -float("inf")
+        k[0, 1, 690:, D - 2] = -float("inf")
+    out = F.attention_fwd(*dev, out_dtype=torch.float32, max_key_splits=splits).cpu().numpy()
+    assert np.isfinite(out).all()
+    assert_bars(norm_error(out, oracle_rows(host))[0], "f32", f"{dt} D{D} infinite keys")
