@@ -283,7 +283,10 @@ def dtype_code(t) -> int:
 
 
 def _raw_stream(torch, device) -> int:
-    """The current stream's handle on a GPU device."""
+    """The current stream's handle on a GPU device; another device is refused here,
+    as torch.cuda.current_stream does (the score tile has no other check of it)."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

@@ -557,6 +557,17 @@ def test_attention_fwd_rejects_mismatched_inputs_before_launch(ofh):
             ofh.attention_fwd(qq, kk, vv, **args)
 
 
+def test_qk_score_tile_refuses_host_tensors(ofh):
+    """A score tile of tensors that are not on the GPU is refused before a pointer
+    reaches the C ABI."""
+    torch = pytest.importorskip("torch")
+    q, k = torch.zeros(1, 4, 8), torch.zeros(1, 5, 8)
+    with pytest.raises(ValueError, match="cuda device"):
+        ofh.qk_score_tile(q, k)
+    with pytest.raises(ValueError, match="cuda device"):
+        ofh.qk_score_tile(q, k, out=torch.zeros(1, 4, 5), bias=torch.zeros(4, 5), scale=0.5)
+
+
 def test_one_hip_runtime_when_the_library_loads_before_torch():
     """Loading the library first must not leave two HIP runtimes in the process
     (torch's bundled copy and /opt/rocm's): the binding imports torch before
