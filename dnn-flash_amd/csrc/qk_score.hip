@@ -22,6 +22,7 @@ namespace ofh {
 namespace {
 
 constexpr int64_t kMaxGridZ = 65535;   // tiles per launch (grid z)
+constexpr int64_t kMaxWorkItems = (int64_t(1) << 32) - 1;  // work items of a launch along x
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T x) { return (float)x; }
@@ -651,7 +652,7 @@ hipError_t launch_qk_score_mfma(const QkScoreArgs& a, int dtype, hipStream_t s) 
                       63 * (a.c_sm + a.c_sn) + 4 < lim31 && a.b_sn >= 0 && a.c_sm >= 0 && a.c_sn >= 0;
     if (rows) {
         const int64_t nqb = (a.M + kMfmaBlock - 1) / kMfmaBlock, nkb = (a.N + kMfmaBlock - 1) / kMfmaBlock;
-        const int64_t max_grid = (int64_t(1) << 31) - 1;
+        const int64_t max_grid = kMaxWorkItems / 256;  // workgroups of a launch
         const bool vec = c_vec && b_vec && a.N % 4 == 0;
         for (int64_t b0 = 0; b0 < a.batch;) {
             QkScoreArgs x = a;

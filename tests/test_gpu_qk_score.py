@@ -289,6 +289,22 @@ def test_batch_beyond_one_launch(ofh, algorithm):
         assert (np.abs(got.astype(np.float64) - want) <= _mfma_bound(uq, uk, 0.5, want)).all()
 
 
+@pytest.mark.parametrize("bias,softcap", [(True, 0.0), (False, 4.0), (False, 0.0)])
+def test_row_kernel_beyond_one_launch(ofh, bias, softcap):
+    """More workgroups of the row kernel than the 2^32 work items of a launch
+    hold: 2^24 + 5 tiles of one score (one query and key, a bias of their own)."""
+    T = (1 << 24) + 5
+    q = torch.full((1, 1, 8), 0.5, device="cuda", dtype=torch.bfloat16).expand(T, 1, 8)
+    k = torch.full((1, 1, 8), 0.25, device="cuda", dtype=torch.bfloat16).expand(T, 1, 8)
+    b = torch.arange(T, device="cuda", dtype=torch.float32).remainder_(1000).view(T, 1, 1) if bias else None
+    out = torch.full((T, 1, 1), -7.0, device="cuda")
+    ofh.qk_score_tile(q, k, bias=b, softcap=softcap, out=out, algorithm=ofh.QK_MFMA)
+    want = torch.ones_like(out) + (b if bias else 0.0)
+    if softcap:
+        want = softcap * torch.tanh(want / softcap)
+    assert (out - want).abs().max().item() <= 2e-6
+
+
 def test_full_size_mfma_against_exact(ofh):
     """Attention-sized tiles (4 heads of 4096 x 4096, d = 128, bf16): the MFMA
     scores stay within the bound of the exact kernel's, and sampled rows match
