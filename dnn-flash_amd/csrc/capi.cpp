@@ -385,6 +385,39 @@ void choose_f32_waves(const ofh_attention_params* p, Resolved& r) {
     r.num_k_tiles = (int)((N + r.block_n - 1) / r.block_n);
 }
 
+// Exact two-pass calls: 32-row blocks of eight wavefronts, or a wavefront per
+// row. A block costs the same for one row as for 32 and for one key as for 256
+// (11-12 us a round of the CUs up to 64 columns, 17 up to 128, 26-34 up to 256),
+// a row a few us of its own and 0.2 us per key, the chip many at once. So rows
+// of few keys, alone or few per head, are faster on their own, everything else
+// in blocks. The estimates are a fit to 740 calls (heads 1-65536, rows 1-400, keys
+// 1-4096, D 20-256, all dtypes): the better kernel's time is missed by 0.5 % on the
+// geometric mean, by a third at most. Measured, wavefront per row / blocks
+// (us): D50 BH65536 M1 N16 377 / 2672, M8 1803 / 2726, M16 3342 / 2844; BH16384
+// M4 N64 691 / 696, M8 1177 / 709; BH4096 M1 N256 586 / 250; D20 BH32 M3 N1 5.1 /
+// 11.5; D75 BH131 M7 N2 9.4 / 17.5; D50 BH2 M1 N64 20.1 / 11.6. Neither takes a
+// grid past the launch range.
+bool rows_in_blocks(const ofh_attention_params* p) {
+    if (p->head_dim > (size_t)ofh::kRowBlockMaxDim || p->value_dim > (size_t)ofh::kRowBlockMaxDim) return false;
+    const int64_t bh = (int64_t)p->batch * p->heads, M = (int64_t)p->query_tokens, N = (int64_t)p->key_tokens;
+    const int64_t rows = bh * M, blocks = bh * ((M + ofh::kRowBlock - 1) / ofh::kRowBlock);
+    if (!ofh::grid_fits(blocks, ofh::kRowBlockThreads)) return false;
+    if (!ofh::grid_fits((rows + ofh::kRowsPerWorkgroup - 1) / ofh::kRowsPerWorkgroup, 64 * ofh::kRowsPerWorkgroup))
+        return true;
+    auto up = [](int64_t x, int64_t y) { return (double)((x + y - 1) / y); };
+    const int64_t keys = p->causal ? std::min(M, N) : N;  // of the longest row
+    const double D = (double)p->head_dim, chunks = up(keys, 64);
+    const double wide = up((int64_t)std::max(p->head_dim, p->value_dim), 64);
+    // a row alone, by the chunks of 64 keys it scores, the keys it sums and the
+    // chunks the causal rule hides; many rows; K and V (a lane walks a K row of
+    // its own, far from the memory's rate); blocks, in rounds of the CUs
+    const double lone = 2.0 + 0.08 * D * chunks + 0.21 * wide * keys + 5.0 * (up(N, 64) - chunks);
+    const double many = 1e-3 * rows * (0.022 * D * chunks + 0.115 * wide * keys);
+    const double read = (double)bh * keys * (double)(p->head_dim + p->value_dim) * elem_size(p->dtype) / 0.52e6;
+    const double block = up(blocks, kComputeUnits) * (3.7 + 9.3 * wide * up(keys, 8 * ofh::kRowBlock));
+    return block <= std::max({lone, many, read});
+}
+
 int resolve(const ofh_attention_params* p, const void* q, const void* k, const void* v,
             const void* out, Resolved& r) {
     contiguous_strides(r.qs, p->q_strides, p->heads, p->query_tokens, p->head_dim);
@@ -429,7 +462,11 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
         r.tile_list = false;
         r.lds_list = false;
         r.paired = false;
-        const bool blocks = ofh::row_blocks_take((int)p->head_dim, (int)p->value_dim);
+        const bool blocks = rows_in_blocks(p);
+        const int64_t bh = (int64_t)p->batch * p->heads, rows = (int64_t)p->query_tokens;
+        if (!blocks && !ofh::grid_fits((bh * rows + ofh::kRowsPerWorkgroup - 1) / ofh::kRowsPerWorkgroup,
+                                       64 * ofh::kRowsPerWorkgroup))
+            return set_error(OFH_ERROR_UNSUPPORTED, "rowwise grid exceeds 2^32 threads");
         r.block_m = blocks ? ofh::kRowBlock : 1;
         r.block_n = blocks ? ofh::kRowBlock : 64;
         r.threads = blocks ? ofh::kRowBlockThreads : 256;
@@ -762,6 +799,7 @@ int fwd_impl(const ofh_attention_params* p, const void* q, const void* k, const 
     if (int rc = resolve(p, q, k, v, out, r)) return rc;
     ofh::FwdArgs a = make_args(p, r, q, k, v, out);
     if (r.algorithm == OFH_ALGO_ROWWISE) {
+        a.split_bm = r.block_m;
         OFH_HIP_CHECK(ofh::launch_rowwise(a, p->dtype, stream));
         return OFH_SUCCESS;
     }

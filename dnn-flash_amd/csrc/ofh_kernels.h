@@ -178,6 +178,11 @@ struct QkScoreArgs {
     int vec4;   // set by the launcher: 16-byte score (and bias) row runs are aligned
 };
 
+// Work items of a launch along x. The runtime cuts a larger grid off without an
+// error, so callers check (an int64 division: the product may not fit).
+constexpr int64_t kMaxWorkItems = (int64_t(1) << 32) - 1;
+inline bool grid_fits(int64_t workgroups, int threads) { return workgroups <= kMaxWorkItems / threads; }
+
 // Launchers; each returns the hipError_t of the launch.
 hipError_t launch_flash_mfma(const FwdArgs& a, int dtype, bool general_mod, hipStream_t s);
 // 16-bit calls whose eight wavefronts split the keys of 256 / groups query rows
@@ -229,13 +234,14 @@ constexpr int kDecodeLoads = 4;
 inline int decode_step_keys(int dtype, int D, int Dv) {
     return kDecodeThreads / 64 * kDecodeLoads * (64 / decode_row_lanes(dtype, D, Dv));
 }
+// Exact two-pass calls: split_bm = kRowBlock runs 32-row blocks of eight
+// wavefronts on the matrix cores (head dims up to kRowBlockMaxDim: Q, and a K or
+// V block per wavefront, in LDS), split_bm = 1 a wavefront per row.
 hipError_t launch_rowwise(const FwdArgs& a, int dtype, hipStream_t s);
-// Exact two-pass calls run 32-row blocks of eight wavefronts on the matrix
-// cores up to these head dims (Q, and a K or V block per wavefront, in LDS),
-// wider heads a wavefront per row.
-inline bool row_blocks_take(int D, int Dv) { return D <= 256 && Dv <= 256; }
 constexpr int kRowBlock = 32;  // query rows per workgroup, keys per wavefront tile
+constexpr int kRowBlockMaxDim = 256;
 constexpr int kRowBlockThreads = 512;
+constexpr int kRowsPerWorkgroup = 4;  // wavefronts (rows) per workgroup of the other kernel
 hipError_t launch_tile_lists(const TileListArgs& a, hipStream_t s);
 // Merge of the key-split partial rows into O in a second launch (num_splits > 1,
 // split_counters null); dtype is the input type.

@@ -22,7 +22,6 @@ namespace ofh {
 namespace {
 
 constexpr int64_t kMaxGridZ = 65535;   // tiles per launch (grid z)
-constexpr int64_t kMaxWorkItems = (int64_t(1) << 32) - 1;  // work items of a launch along x
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T x) { return (float)x; }

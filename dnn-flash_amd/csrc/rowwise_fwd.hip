@@ -8,17 +8,16 @@
 // unaligned rows).
 //
 // rowwise_fwd_kernel (head_dim and value_dim up to 256): 32 query rows per
-// workgroup on the fp32 matrix cores. rowwise_wide_kernel (wider heads): one
-// wavefront per query row on the vector units.
+// workgroup on the fp32 matrix cores. rowwise_wave_kernel (wider heads, and few
+// rows per head against few keys): one wavefront per query row on the vector units.
 
 #include "ofh_kernels.h"
 
 namespace ofh {
 namespace {
 
-constexpr int kRowsPerBlock = 4;   // rowwise_wide_kernel: one wavefront per query row
-constexpr int kMaxD = 1024;        // ... its query row staged in LDS (fp32)
-constexpr int kAccPerLane = 8;     // ... output columns per lane per pass-2 sweep (512 per sweep)
+constexpr int kMaxD = 1024;     // rowwise_wave_kernel: its query row staged in LDS (fp32)
+constexpr int kAccPerLane = 8;  // ... output columns per lane per pass-2 sweep (512 per sweep)
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T x) {
@@ -47,15 +46,19 @@ __device__ __forceinline__ float row_score(const FwdArgs& a, const float* qs, co
     return s;
 }
 
-// Heads wider than rowwise_fwd_kernel takes. Lanes own keys during the score
-// passes (each lane one key, the query row broadcast from LDS) and own output
+// Heads wider than rowwise_fwd_kernel takes, and calls that give its 32-row
+// blocks little to do: a wavefront here costs a fraction of a block whose
+// eight wavefronts stage 32 rows and 32 keys whatever is there (fp32 D50 B1024
+// H64 M1 N16 377 us against 2672, one row of three keys 5.1 us against 11.2).
+// What bounds it: the latency of the loads behind one another, one per key in
+// pass 2. Lanes own keys during the score passes (each lane one key, the query row broadcast from LDS) and own output
 // columns during accumulation (each of the 64 probabilities of a key chunk is
 // broadcast with a scalar read-lane), so V reads are coalesced along the row.
 template <typename T>
-__global__ __launch_bounds__(64 * kRowsPerBlock) void rowwise_wide_kernel(FwdArgs a) {
-    __shared__ float qs_all[kRowsPerBlock][kMaxD];
+__global__ __launch_bounds__(64 * kRowsPerWorkgroup) void rowwise_wave_kernel(FwdArgs a) {
+    __shared__ float qs_all[kRowsPerWorkgroup][kMaxD];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t row_id = (int64_t)blockIdx.x * kRowsPerBlock + w;
+    const int64_t row_id = (int64_t)blockIdx.x * kRowsPerWorkgroup + w;
     const bool valid = row_id < (int64_t)a.B * a.H * a.M;  // wave-uniform
     const int qi = valid ? (int)(row_id % a.M) : 0;
     const int bh = valid ? (int)(row_id / a.M) : 0;
@@ -444,15 +447,16 @@ hipError_t launch_row_blocks(const FwdArgs& a, hipStream_t s) {
 
 template <typename T>
 hipError_t launch_rowwise_t(const FwdArgs& a, hipStream_t s) {
-    if (row_blocks_take(a.D, a.Dv)) {
+    if (a.split_bm == kRowBlock) {
+        if (a.D > kRowBlockMaxDim || a.Dv > kRowBlockMaxDim) return hipErrorInvalidValue;
         constexpr int NW = kRowWaves;
         if (a.Dv <= 64) return launch_row_blocks<T, NW, 1>(a, s);
         if (a.Dv <= 128) return launch_row_blocks<T, NW, 2>(a, s);
         return launch_row_blocks<T, NW, 4>(a, s);
     }
     const int64_t rows = (int64_t)a.B * a.H * a.M;
-    hipLaunchKernelGGL(rowwise_wide_kernel<T>, dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
-                       dim3(64 * kRowsPerBlock), 0, s, a);
+    hipLaunchKernelGGL(rowwise_wave_kernel<T>, dim3((unsigned)((rows + kRowsPerWorkgroup - 1) / kRowsPerWorkgroup)),
+                       dim3(64 * kRowsPerWorkgroup), 0, s, a);
     return hipGetLastError();
 }
 

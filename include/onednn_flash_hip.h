@@ -71,7 +71,8 @@ typedef enum ofh_bias_kind {
  * against many keys (decoding: no mask, bias, soft-cap or causal rule) run on
  * a vector kernel. ROWWISE is the exact two-pass softmax of
  * standard_attention, run on the GPU in 32-row blocks up to head_dim and
- * value_dim 256 and one query row per wavefront above. */
+ * value_dim 256, and one query row per wavefront above and for a few rows per
+ * head against few keys. */
 typedef enum ofh_algorithm {
     OFH_ALGO_AUTO = 0,
     OFH_ALGO_FLASH_MFMA = 1,

@@ -451,6 +451,37 @@ def test_f32_waves_choice(ofh):
         assert "waves" not in other, other
 
 
+def test_rowwise_choice(ofh):
+    """Exact two-pass calls: a wavefront per row for few rows per head against
+    few keys and for heads wider than 256, 32-row blocks for the others; never a
+    grid of 2^32 threads or more, which a launch would cut off."""
+    F = ofh
+
+    def info(B, H, M, N, D, **kw):
+        return F.launch_info(F.make_params(B, H, M, N, D, algorithm=F.ALGO_ROWWISE, **kw))
+
+    for call in [(1024, 64, 1, 16, 50), (1, 1, 1, 1, 64), (1, 32, 3, 1, 20), (256, 64, 2, 40, 50), (1, 131, 7, 2, 75),
+                 (1, 8, 300, 200, 257), (1, 64, 11, 8, 64, 300)]:
+        i = info(*call[:5], **(dict(value_dim=call[5]) if len(call) > 5 else {}))
+        assert i.block_m == 1 and i.threads == 256 and i.workgroups == (call[0] * call[1] * call[2] + 3) // 4, call
+    for call in [(2, 8, 1024, 1024, 64), (1, 4, 100, 1000, 50), (1, 2, 1, 4096, 64), (64, 64, 4, 256, 50), (1, 2, 33, 300, 256),
+                 (1024, 64, 32, 16, 50)]:
+        i = info(*call)
+        assert i.block_m == 32 and i.threads == 512 and i.workgroups == call[0] * call[1] * ((call[2] + 31) // 32), call
+    for bh in [1 << 21, (1 << 23) - 1, 1 << 23, (1 << 24) + 3, (1 << 26) - 4]:
+        for M in [1, 2, 7, 8, 31, 33, 64]:
+            for N in [1, 40, 300]:
+                for causal in [False, True]:
+                    try:
+                        i = info(1, bh, M, N, 16, causal=causal)
+                    except RuntimeError:
+                        assert bh * M >= (1 << 26) - 4 and bh * ((M + 31) // 32) >= 1 << 23
+                        continue
+                    assert i.workgroups * i.threads < 1 << 32, (bh, M, N)
+    p = F.make_params(1, 1 << 27, 1, 40, 16, algorithm=F.ALGO_ROWWISE)
+    _expect_error(F, p, F.OFH_ERROR_UNSUPPORTED, "rowwise grid")
+
+
 def test_flat_params_layout(ofh):
     """attention_fwd's positionally built parameters are byte for byte the
     ofh_attention_params that make_params fills."""

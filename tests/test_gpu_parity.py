@@ -322,6 +322,25 @@ def test_rowwise_row_blocks(ofh, dt, D, Dv):
     assert_bars(norm_error(out[finite], want[finite])[0], dt, "finite rows beside non-finite V")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("H,M,N,D,Dv", [(1, 1, 1, 1, 1), (3, 1, 5, 20, 33), (70, 3, 7, 75, 50), (600, 2, 37, 50, 130),
+                                        (2000, 5, 9, 33, 33), (40, 4, 12, 256, 200)])
+def test_rowwise_few_rows(ofh, dt, H, M, N, D, Dv):
+    """Few rows per head against few keys (a wavefront per row), in [B,T,H,D]
+    storage: plain, causal with ALiBi and a soft-cap, with a block mask that
+    hides some rows' keys, and with a dense bias."""
+    dev, host = make_inputs(dt, 1, H, M, N, D, Dv, seed=H)
+    info = ofh.launch_info(ofh.make_params(1, H, M, N, D, Dv, algorithm=ofh.ALGO_ROWWISE))
+    assert info.block_m == 1
+    dev = tuple(t.transpose(1, 2).contiguous().transpose(1, 2) for t in dev)
+    slopes, bias = alibi_slopes(H), O.normal(5, (M, N))
+    mask = np.ones((2, 2), np.uint8)
+    mask[0, 0] = 0
+    for kw in [dict(), dict(causal=True, slopes=slopes, softcap=20.0), dict(mask=mask, mbs=(2, 4)), dict(bias=bias)]:
+        out = run(ofh, dev, dt=dt, algorithm=ofh.ALGO_ROWWISE, **kw)
+        check(out, oracle_full(host, **kw), dt, f"{dt} a wavefront per row H{H} M{M} N{N} D{D} Dv{Dv} {sorted(kw)}")
+
+
 def test_strided_layouts(ofh):
     B, H, M, N, D = 2, 4, 150, 170, 128
     dev, host = make_inputs("bf16", B, H, M, N, D, seed=13)
