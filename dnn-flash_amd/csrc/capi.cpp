@@ -385,6 +385,21 @@ void choose_f32_waves(const ofh_attention_params* p, Resolved& r) {
     r.num_k_tiles = (int)((N + r.block_n - 1) / r.block_n);
 }
 
+// fp32 calls of three to eight rows whose heads alone do not fill the CUs: the 16-
+// and 32-row blocks, which multiply on the matrix cores, end sooner than the
+// decode kernel while the keys are few. That one holds 4 or 8 rows, whatever the
+// call has. Measured, blocks / decode kernel (us): D32 M8 BH11 N241 5.2 / 8.9, BH3
+// M5 N421 6.6 / 11.0, BH15 M8 N1063 11.0 / 12.3, BH8 M6 N4323 12.3 / 13.9, BH125 M6
+// N3609 36.6 / 33.4; D64 M8 BH11 N631 10.2 / 12.1, M5 BH1 N765 11.4 / 10.9, M6 BH10
+// N1091 14.0 / 12.3. Up to four rows: D32 N360 5.8 / 6.6, N676 8.5 / 8.9, N1094 10.6
+// / 8.5; D64 N166 6.2 / 6.1, N234 6.1 / 6.8, N456 9.2 / 8.3, with over 64 heads (two
+// splits of the keys at most) BH104 N284 7.9 / 9.6.
+bool decode_rows_on_blocks(const ofh_attention_params* p, int kdim) {
+    const int64_t bh = (int64_t)p->batch * p->heads, M = (int64_t)p->query_tokens, N = (int64_t)p->key_tokens;
+    if (p->dtype != OFH_DTYPE_F32 || kdim > 64 || bh >= ofh::kRows32Below || M <= 2) return false;
+    return N <= (kdim == 32 ? (M <= 4 ? 1024 : 4096) : (M > 4 ? 1024 : bh > 64 ? 512 : 256));
+}
+
 // Exact two-pass calls: 32-row blocks of eight wavefronts, or a wavefront per
 // row. A block costs the same for one row as for 32 and for one key as for 256
 // (11-12 us a round of the CUs up to 64 columns, 17 up to 128, 26-34 up to 256),
@@ -500,7 +515,9 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     // that streams K and V through registers. Planned as one 32-row query
     // block per head. (2^30: its key positions are 32-bit sums.)
     r.decode = p->algorithm == OFH_ALGO_AUTO && !r.tile_list && !r.general_mod && !p->causal &&
-               (int64_t)p->query_tokens <= ofh::decode_max_rows(p->dtype, (int)p->head_dim, (int)p->value_dim) && p->key_tokens >= (size_t)ofh::kDecodeMinKeys && p->key_tokens <= (size_t)1 << 30;
+               (int64_t)p->query_tokens <= ofh::decode_max_rows(p->dtype, (int)p->head_dim, (int)p->value_dim) &&
+               p->key_tokens >= (size_t)ofh::kDecodeMinKeys && p->key_tokens <= (size_t)1 << 30 &&
+               !decode_rows_on_blocks(p, r.kdim);
     if (r.decode) {
         r.block_m = 32;
         r.block_n = ofh::decode_step_keys(p->dtype, (int)p->head_dim, (int)p->value_dim);

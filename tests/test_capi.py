@@ -269,7 +269,21 @@ def test_kernel_choice(ofh):
         (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=264), "rowwise_fwd_kernel"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, algorithm=F.ALGO_ROWWISE), "rowwise_fwd_kernel"),
         # a few query rows (8 fp32, 2 16-bit), plain scale, no mask: the decode kernel
-        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 8, 200)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 64, 8, 200)), "flash_fwd_decode_kernel<f32,64>"),
+        # ... fp32 with three rows or more, few heads and few keys: the 16-row blocks
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 8, 200)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 127, 5, 1024)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 128, 5, 1024)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 8, 5, 1025)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 8, 4, 256)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 8, 4, 257)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 65, 4, 512)), "flash_fwd_f32_rows16_kernel<64,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 65, 4, 513)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(1, 8, 2, 64)), "flash_fwd_decode_kernel<f32,64>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=32, shape=(1, 8, 3, 1024)), "flash_fwd_f32_rows16_kernel<32,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=32, shape=(1, 8, 3, 1025)), "flash_fwd_decode_kernel<f32,32>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=32, shape=(1, 8, 8, 4096)), "flash_fwd_f32_rows32_kernel<32,plain>"),
+        (dict(dtype=F.DTYPE_F32, head_dim=80, shape=(1, 8, 8, 64)), "flash_fwd_decode_kernel<f32,128>"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 3, 9, 200)), "flash_fwd_f32_rows16_kernel<64,plain>"),
         (dict(dtype=F.DTYPE_BF16, head_dim=80, shape=(2, 3, 2, 200)), "flash_fwd_decode_kernel<bf16,128>"),
         (dict(dtype=F.DTYPE_F16, head_dim=64, value_dim=128, shape=(2, 3, 1, 200)), "flash_fwd_decode_kernel<f16,128>"),
