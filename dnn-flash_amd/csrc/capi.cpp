@@ -433,6 +433,11 @@ bool rows_in_blocks(const ofh_attention_params* p) {
     return block <= std::max({lone, many, read});
 }
 
+// Workgroups of the MFMA and decode kernels' launch.
+int64_t workgroups_of(const ofh_attention_params* p, const Resolved& r) {
+    return (int64_t)p->batch * p->heads * (r.paired ? (r.num_q_tiles + 1) / 2 : r.num_q_tiles) * r.key_splits;
+}
+
 int resolve(const ofh_attention_params* p, const void* q, const void* k, const void* v,
             const void* out, Resolved& r) {
     contiguous_strides(r.qs, p->q_strides, p->heads, p->query_tokens, p->head_dim);
@@ -517,7 +522,7 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     r.decode = p->algorithm == OFH_ALGO_AUTO && !r.tile_list && !r.general_mod && !p->causal &&
                (int64_t)p->query_tokens <= ofh::decode_max_rows(p->dtype, (int)p->head_dim, (int)p->value_dim) &&
                p->key_tokens >= (size_t)ofh::kDecodeMinKeys && p->key_tokens <= (size_t)1 << 30 &&
-               !decode_rows_on_blocks(p, r.kdim);
+               !decode_rows_on_blocks(p, r.kdim) && ofh::grid_fits((int64_t)p->batch * p->heads, ofh::kDecodeThreads);
     if (r.decode) {
         r.block_m = 32;
         r.block_n = ofh::decode_step_keys(p->dtype, (int)p->head_dim, (int)p->value_dim);
@@ -570,6 +575,8 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
     choose_key_groups(p, r);
     choose_f32_waves(p, r);
     set_lds_list(p, r);
+    if (!ofh::grid_fits(workgroups_of(p, r), r.threads))
+        return set_error(OFH_ERROR_UNSUPPORTED, "grid exceeds 2^32 threads");
     return OFH_SUCCESS;
 }
 
@@ -1126,8 +1133,7 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
         info->block_m = r.block_m;
         info->block_n = r.block_n;
         info->threads = r.threads;
-        info->workgroups = (int64_t)p->batch * p->heads * (r.paired ? (r.num_q_tiles + 1) / 2 : r.num_q_tiles) *
-                           r.key_splits;
+        info->workgroups = workgroups_of(p, r);
         info->key_splits = r.key_splits;
         info->merge_in_launch = merge_in_launch(p, r) ? 1 : 0;
         name = r.decode ? decode_kernel_name(p->dtype, (int)p->head_dim, (int)p->value_dim)

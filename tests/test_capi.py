@@ -465,6 +465,29 @@ def test_f32_waves_choice(ofh):
         assert "waves" not in other, other
 
 
+def test_grids_fit_a_launch(ofh):
+    """No plan has 2^32 threads or more (a launch would cut it off without an
+    error): fp32 decoding keeps the heads that other kernels serve with smaller
+    workgroups, what no kernel holds is refused."""
+    F = ofh
+    for dtype, threads in [(F.DTYPE_F32, 256), (F.DTYPE_BF16, 512), (F.DTYPE_F16, 512)]:
+        for heads in [1 << 20, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, 1 << 30]:
+            for M, N, kw in [(1, 64, {}), (1, 300, dict(softcap=5.0)), (2, 64, dict(causal=True)), (300, 300, {})]:
+                p = F.make_params(1, heads, M, N, 64, dtype=dtype, **kw)
+                if heads * ((M + 127) // 128) * threads >= 1 << 34:
+                    _expect_error(F, p, F.OFH_ERROR_UNSUPPORTED, "grid exceeds")
+                    continue
+                try:
+                    i = F.launch_info(p)
+                except RuntimeError as e:
+                    assert "grid exceeds" in str(e) and heads * ((M + 127) // 128) * threads >= 1 << 32
+                    continue
+                assert i.workgroups * i.threads < 1 << 32
+    info = F.launch_info(F.make_params(1, (1 << 24) - 1, 1, 64, 64, dtype=F.DTYPE_F32))
+    assert info.threads == 256 and not info.kernel_name.decode().startswith("flash_fwd_decode_kernel")
+    assert F.launch_info(F.make_params(1, (1 << 23) - 1, 1, 64, 64)).kernel_name.decode().startswith("flash_fwd_decode_kernel")
+
+
 def test_rowwise_choice(ofh):
     """Exact two-pass calls: a wavefront per row for few rows per head against
     few keys and for heads wider than 256, 32-row blocks for the others; never a
