@@ -390,7 +390,7 @@ enum QkPost { QK_POST_NONE = 0, QK_POST_BIAS = 1, QK_POST_CAP = 2, QK_POST_BIAS_
 // 4 bytes, whole 256-byte row pieces as well. Measured (us, one-block kernel ->
 // this): bf16 32 tiles 2048^2 x 128 with a shared bias 209 -> 169 (3.5 TB/s), with
 // a bias per tile, 16 tiles, 148 -> 110 (4.9 TB/s), with a soft-cap 200 -> 169; 30
-// tiles 1001 x 1003 x 64, shared bias 69 -> 52, no bias 55 -> 42. A shared bias
+// tiles 1001 x 1003 x 64, shared bias 69 -> 47, no bias 55 -> 33. A shared bias
 // with the tiles of an XCD one after another (the order of the other calls):
 // 182.
 constexpr int kRowBufBytes = 32 * 1024;   // one K block (128 rows x 16 CH bytes), or the epilogue staging
@@ -573,18 +573,32 @@ __global__ __launch_bounds__(256, 2) void qk_score_mfma_rows_kernel(QkScoreArgs 
                     for (int it = 0; it < 8; ++it) rows4(it);
                 }
             } else {
-                auto row1 = [&](int row) {
-                    const int rr = 32 * x + row;
-                    if (i0 + rr >= a.M || j0 + lane >= a.N) return;
-                    const float raw = *(const qk_lds_f32*)(stg + row * 256 + 16 * ((lane >> 2) ^ (row & 15)) + 4 * (lane & 3));
-                    cw[rr * csm + lane * csn] = post(raw, BIASED ? bias[row] : 0.0f);
+                // Eight rows at a time are read before the first is stored: a row that is
+                // read under its own bounds check waits for its LDS read alone (9 tiles 230 x
+                // 110 x 128 9.8 us so, 7.7 now). Rows past the end hold products that are not
+                // stored.
+                const int rows = (int)min((int64_t)32, a.M - i0 - 32 * x);  // uniform
+                const bool in_col = j0 + lane < a.N;
+                auto rows8 = [&](int r0) {
+                    if (r0 >= rows) return;
+                    float v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        v[u] = *(const qk_lds_f32*)(stg + (r0 + u) * 256 + 16 * ((lane >> 2) ^ ((r0 + u) & 15)) + 4 * (lane & 3));
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = post(v[u], BIASED ? bias[r0 + u] : 0.0f);
+                    if (!in_col) return;
+                    float* cr = cw + ((32 * x + r0) * csm + lane * csn);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (r0 + u < rows) cr[u * csm] = v[u];
                 };
                 if constexpr (BIASED) {
 #pragma unroll
-                    for (int row = 0; row < 32; ++row) row1(row);
+                    for (int r0 = 0; r0 < 32; r0 += 8) rows8(r0);
                 } else {
-#pragma unroll 4
-                    for (int row = 0; row < 32; ++row) row1(row);
+#pragma unroll 1
+                    for (int r0 = 0; r0 < 32; r0 += 8) rows8(r0);
                 }
             }
             if constexpr (BIASED) {
