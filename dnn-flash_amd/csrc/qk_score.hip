@@ -621,6 +621,23 @@ inline int64_t rows_blocks_per_workgroup(int64_t tiles, int64_t nkb) {
     return std::min(tpw, nkb);
 }
 
+// Soft-capped calls are bound by the vector ALU, so the time is that of the
+// busiest CU: rounds of two runs of blocks (row kernel) or of three blocks
+// (one-block kernel, whose third workgroup per CU hides less else). Where the
+// runs leave more of their last round empty, the one-block kernel is faster.
+// Measured, one-block / row kernel (us): 11 tiles 924 x 988 x 32, 704 blocks, 17.4 /
+// 20.2; 63 tiles 1122 x 48 x 128 with a bias, 567 blocks, 18.8 / 24.8; 35 tiles 645 x
+// 776 x 64, 1470 blocks, 31.7 / 37.0; against 56 tiles 241 x 1092 x 16 with a bias,
+// 1008 blocks, 29.5 / 24.0; 12 tiles 1363 x 372 x 64, 396 blocks, 15.3 / 14.3. (Without
+// 16-byte rows the row kernel is faster throughout.)
+inline bool block_kernel_fills_better(int64_t batch, int64_t nqb, int64_t nkb) {
+    const int64_t blocks = batch * nqb * nkb, tpw = rows_blocks_per_workgroup(blocks, nkb);
+    const int64_t runs = batch * nqb * ((nkb + tpw - 1) / tpw);
+    const int64_t run_rounds = (runs + 2 * kComputeUnits - 1) / (2 * kComputeUnits);
+    const int64_t block_rounds = (blocks + 3 * kComputeUnits - 1) / (3 * kComputeUnits);
+    return 3 * block_rounds < 2 * tpw * run_rounds;
+}
+
 template <typename T, int CH, int POST>
 void launch_rows_post(const QkScoreArgs& x, bool vec, int64_t nqb, int64_t npieces, int tpw, hipStream_t s) {
     const dim3 grid((unsigned)(x.batch * nqb * npieces));
@@ -663,10 +680,10 @@ hipError_t launch_qk_score_mfma(const QkScoreArgs& a, int dtype, hipStream_t s) 
     const int64_t lim31 = int64_t(1) << 31;
     const bool rows = a.K <= 128 && (kMfmaBlock - 1) * a.b_sn + a.K < lim31 &&
                       63 * (a.c_sm + a.c_sn) + 4 < lim31 && a.b_sn >= 0 && a.c_sm >= 0 && a.c_sn >= 0;
-    if (rows) {
-        const int64_t nqb = (a.M + kMfmaBlock - 1) / kMfmaBlock, nkb = (a.N + kMfmaBlock - 1) / kMfmaBlock;
+    const int64_t nqb = (a.M + kMfmaBlock - 1) / kMfmaBlock, nkb = (a.N + kMfmaBlock - 1) / kMfmaBlock;
+    const bool vec = c_vec && b_vec && a.N % 4 == 0;
+    if (rows && !(a.softcap > 0.0f && vec && block_kernel_fills_better(a.batch, nqb, nkb))) {
         const int64_t max_grid = kMaxWorkItems / 256;  // workgroups of a launch
-        const bool vec = c_vec && b_vec && a.N % 4 == 0;
         for (int64_t b0 = 0; b0 < a.batch;) {
             QkScoreArgs x = a;
             x.batch = std::min<int64_t>(a.batch - b0, std::max<int64_t>(1, max_grid / (nqb * nkb)));

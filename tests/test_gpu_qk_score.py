@@ -289,6 +289,20 @@ def test_batch_beyond_one_launch(ofh, algorithm):
         assert (np.abs(got.astype(np.float64) - want) <= _mfma_bound(uq, uk, 0.5, want)).all()
 
 
+@pytest.mark.parametrize("T", [512, 567, 769])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_softcap_by_number_of_blocks(ofh, T, with_bias):
+    """Soft-capped calls of 513 to 768 blocks run the one-block kernel, those around
+    them the row kernel: the same scores as the exact kernel's within the bound of
+    another summation order (the cap's slope is at most 1), plus tanh's error."""
+    (q, uq), (k, uk) = (to_device(O.normal(T + i, (T, n, 72)), "bf16") for i, n in ((0, 20), (1, 24)))
+    bias = _dev32(O.normal(9, (20, 24))) if with_bias else None
+    kw = dict(scale=0.125, bias=bias, softcap=3.0)
+    got = _run(ofh, q, k, algorithm=ofh.QK_MFMA, **kw).cpu().numpy()
+    want = _run(ofh, q, k, algorithm=ofh.QK_EXACT, **kw).cpu().numpy()
+    assert (np.abs(got - want) <= _mfma_bound(uq, uk, 0.125, want) + 2e-6 * np.abs(want)).all()
+
+
 @pytest.mark.parametrize("bias,softcap", [(True, 0.0), (False, 4.0), (False, 0.0)])
 def test_row_kernel_beyond_one_launch(ofh, bias, softcap):
     """More workgroups of the row kernel than the 2^32 work items of a launch
