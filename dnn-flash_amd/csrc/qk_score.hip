@@ -753,13 +753,21 @@ hipError_t launch_qk_score(const QkScoreArgs& a, int dtype, hipStream_t s) {
         x.c = a.c + b0 * a.c_sb;
         if (a.bias != nullptr) x.bias = a.bias + b0 * a.bias_sb;
         x.vec4 = a.c_sn == 1 && a.c_sm % 4 == 0 && a.c_sb % 4 == 0 && (reinterpret_cast<uintptr_t>(a.c) & 15u) == 0;
-        // 64x64 blocks where they give every CU three, 32x32 below (us, 32x32 /
-        // 64x64: 16 tiles 512^2 x 64, 1024 blocks, 24.4 / 20.3; 8 tiles 333 x 777 x
-        // 100, 624 blocks, 24.0 / 25.4; 20 tiles 250 x 430 x 64, 560 blocks, 16.4 /
-        // 18.6; 4 tiles 128^2 x 64, 16 blocks, 5.6 / 10.2). 128x128 blocks gained
+        // 64x64 blocks where they give every CU three or more, for a short k (their
+        // prologue and epilogue weigh more; a bias doubles what the epilogue waits for) many
+        // more, and where they pad little more than 32x32 ones, which take every other call
+        // (us, 32x32 / 64x64: 16 tiles 512^2 x 64, 1024 blocks, 24.4 / 20.3; 15 x 332 x 508 x
+        // 128, 720, 30.5 / 27.4; 5 x 753 x 605 x 64, 600, 15.8 / 17.2; 10 x 707 x 538 x 32, 1080,
+        // 14.3 / 17.6; 24 x 321 x 1656 x 32, 3744, 41.1 / 36.9; 57 x 317 x 1020 x 16, 4560, 40.2 /
+        // 29.6; with a bias 20 x 288 x 797 x 64, 1300, 29.4 / 33.9, 31 x 887 x 896 x 48, 6076,
+        // 98.4 / 78.7; 57 x 1193 x 22 x 24, twice the padding, 10.3 / 18.8). 128x128 blocks gained
         // 1 % at 32 tiles 1024^2 x 128 and lost 35 % at 8 tiles 1100^2 x 96.
         const int64_t blocks64 = x.batch * ((x.M + 63) / 64) * ((x.N + 63) / 64);
-        const hipError_t e = blocks64 >= 3 * kComputeUnits ? launch_qk_exact<4>(x, dtype, s) : launch_qk_exact<2>(x, dtype, s);
+        const int64_t blocks32 = x.batch * ((x.M + 31) / 32) * ((x.N + 31) / 32);
+        const int64_t k = std::min<int64_t>(x.K, 128);
+        const bool wide = blocks64 >= 3 * kComputeUnits && blocks64 * k >= (x.bias != nullptr ? 96 * 1024 : 48 * 1024) &&
+                          200 * blocks64 <= 63 * blocks32;  // 1.26 times the area
+        const hipError_t e = wide ? launch_qk_exact<4>(x, dtype, s) : launch_qk_exact<2>(x, dtype, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

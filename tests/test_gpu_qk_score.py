@@ -123,10 +123,11 @@ def test_mfma_post_ops_at_block_edges(ofh, dt, T, M, N, K):
 
 
 @pytest.mark.parametrize("dt", ["f32", "f16"])
-@pytest.mark.parametrize("T,M,N,K", [(200, 65, 129, 33), (1100, 63, 40, 5), (3, 65, 129, 33), (2, 31, 33, 31)])
+@pytest.mark.parametrize("T,M,N,K", [(200, 65, 129, 33), (1100, 63, 40, 5), (3, 65, 129, 33), (2, 31, 33, 31),
+                                     (60, 257, 190, 65), (140, 125, 190, 129)])
 def test_exact_kernel_block_edges(ofh, dt, T, M, N, K):
-    """Both block sizes of the exact kernel (64x64 from 768 blocks up) past their
-    row, column and k-chunk edges, with either axis of Q and K contiguous: bit
+    """Both block sizes of the exact kernel (the last two shapes run 64x64 ones)
+    past their row, column and k-chunk edges, with either axis of Q and K contiguous: bit
     for bit the oracle's."""
     rng = np.random.default_rng(T + K)
     tq, uq = to_device(rng.standard_normal((T, M, K), dtype=np.float32), dt)
