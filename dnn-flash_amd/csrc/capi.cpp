@@ -517,14 +517,14 @@ int resolve(const ofh_attention_params* p, const void* q, const void* k, const v
         r.staged_bias = ofh::bias_can_be_staged(p->bias, (int64_t)p->key_tokens, bs[0], bs[1], bs[2]);
     }
     // A few query rows (decoding), plain scale and no mask: the vector kernel
-    // that streams K and V through registers. Planned as one 32-row query
-    // block per head. (2^30: its key positions are 32-bit sums.)
+    // that streams K and V through registers, all rows of a head in one
+    // workgroup. (2^30: its key positions are 32-bit sums.)
     r.decode = p->algorithm == OFH_ALGO_AUTO && !r.tile_list && !r.general_mod && !p->causal &&
                (int64_t)p->query_tokens <= ofh::decode_max_rows(p->dtype, (int)p->head_dim, (int)p->value_dim) &&
                p->key_tokens >= (size_t)ofh::kDecodeMinKeys && p->key_tokens <= (size_t)1 << 30 &&
                !decode_rows_on_blocks(p, r.kdim) && ofh::grid_fits((int64_t)p->batch * p->heads, ofh::kDecodeThreads);
     if (r.decode) {
-        r.block_m = 32;
+        r.block_m = ofh::decode_held_rows((int)p->query_tokens);
         r.block_n = ofh::decode_step_keys(p->dtype, (int)p->head_dim, (int)p->value_dim);
         r.threads = ofh::kDecodeThreads;
         r.paired = false;
@@ -1188,7 +1188,7 @@ int ofh_attention_launch_info(const ofh_attention_params* p, ofh_launch_info* in
                                ? ((int64_t)p->batch * p->heads * p->query_tokens + 3) / 4
                                : (int64_t)p->batch * p->heads * (((int64_t)p->query_tokens + r.block_m - 1) / r.block_m);
         info->key_splits = 1;
-        name = "rowwise_fwd_kernel";
+        name = r.block_m == 1 ? "rowwise_wave_kernel" : "rowwise_fwd_kernel";
     }
     std::strncpy(info->kernel_name, name, sizeof(info->kernel_name) - 1);
     return OFH_SUCCESS;

@@ -218,6 +218,8 @@ constexpr int kDecodeThreads = 512;
 inline int decode_max_rows(int dtype, int D, int Dv) {
     return dtype == DT_F32 ? 8 : D <= 128 && Dv <= 128 ? 2 : 0;
 }
+// Query rows the kernel holds for a call of M (its instantiations).
+inline int decode_held_rows(int M) { return M <= 2 ? M : M <= 4 ? 4 : 8; }
 // Fewer keys are no stream: such calls take a launch's latency on any kernel.
 constexpr int kDecodeMinKeys = 64;
 // Lanes that hold a K or V row of the decode kernel, 16 bytes each.

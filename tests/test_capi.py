@@ -261,12 +261,18 @@ def test_kernel_choice(ofh):
         (dict(dtype=F.DTYPE_BF16, head_dim=192, value_dim=128, softcap=5.0), "flash_fwd_lockstep_kernel<bf16,192,mod,4w>"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=48), "flash_fwd_f32_rows16_kernel<64,plain>"),
         (dict(dtype=F.DTYPE_F32, head_dim=40, shape=(8, 16, 1024, 300)), "flash_fwd_mfma32_kernel<64,plain>"),
-        # not a multiple of the 16-byte row chunk, or beyond the kernels' head dims: rowwise
+        # not a multiple of the 16-byte row chunk: 32-row blocks of the rowwise
+        # kernel; beyond the kernels' head dims: a wavefront per row
         (dict(dtype=F.DTYPE_BF16, head_dim=20), "rowwise_fwd_kernel"),
         (dict(dtype=F.DTYPE_F32, head_dim=6), "rowwise_fwd_kernel"),
-        (dict(dtype=F.DTYPE_BF16, head_dim=264), "rowwise_fwd_kernel"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=264), "rowwise_wave_kernel"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=255), "rowwise_fwd_kernel"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=257), "rowwise_wave_kernel"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=20, value_dim=256), "rowwise_fwd_kernel"),
+        (dict(dtype=F.DTYPE_BF16, head_dim=20, value_dim=257), "rowwise_wave_kernel"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, algorithm=F.ALGO_ROWWISE, shape=(64, 64, 1, 8)), "rowwise_wave_kernel"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=160), "flash_fwd_mfma32_kernel<160,plain>"),
-        (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=264), "rowwise_fwd_kernel"),
+        (dict(dtype=F.DTYPE_F32, head_dim=64, value_dim=264), "rowwise_wave_kernel"),
         (dict(dtype=F.DTYPE_F32, head_dim=64, algorithm=F.ALGO_ROWWISE), "rowwise_fwd_kernel"),
         # a few query rows (8 fp32, 2 16-bit), plain scale, no mask: the decode kernel
         (dict(dtype=F.DTYPE_F32, head_dim=64, shape=(2, 64, 8, 200)), "flash_fwd_decode_kernel<f32,64>"),
@@ -313,9 +319,8 @@ def test_kernel_choice(ofh):
     # one round of 128-row pairs or fewer: 128-row tiles (which then split their keys)
     info = F.launch_info(F.make_params(1, 8, 2048, 2048, 192, dtype=F.DTYPE_BF16, causal=True))
     assert info.block_m == 128 and info.threads == 256 and info.key_splits > 1
-    # 16-bit decode: 8 heads x 1 query tile -> 256 staged 128-key tiles per head
-    # in 32 splits of 8: 256 workgroups, one round of the 256 CUs (one
-    # 8-wavefront workgroup per CU)
+    # 16-bit decode: 8 heads -> 256 steps of 128 keys per head in 32 splits of 8:
+    # 256 workgroups, one round of the 256 CUs
     info = F.launch_info(F.make_params(1, 8, 1, 32768, 128, dtype=F.DTYPE_BF16))
     assert info.key_splits == 32 and info.workgroups == 8 * 32
     assert F.launch_info(F.make_params(1, 8, 1, 32768, 128, dtype=F.DTYPE_BF16,
@@ -369,9 +374,13 @@ def test_kernel_choice(ofh):
     assert info.block_m == 32 and info.block_n == 32 and info.threads == 256
     assert info.key_splits == 8 and info.workgroups == 4 * 16 * 8 and info.merge_in_launch == 1
     assert F.workspace_bytes(p) >= 8 * 4 * 512 * 66 * 4
-    # fp32 decode: one 32-row block per head, its 1024 tiles over 32 workgroups
+    # fp32 decode: one workgroup per head holds its rows (1, 2, 4 or 8), the
+    # head's 512 steps of 64 keys over 32 workgroups
+    for M, held in [(1, 1), (2, 2), (3, 4), (4, 4), (5, 8), (8, 8)]:
+        info = F.launch_info(F.make_params(1, 8, M, 32768, 128, dtype=F.DTYPE_F32))
+        assert info.block_m == held and info.block_n == 64
     info = F.launch_info(F.make_params(1, 8, 1, 32768, 128, dtype=F.DTYPE_F32))
-    assert info.block_m == 32 and info.key_splits == 32 and info.workgroups == 8 * 32
+    assert info.key_splits == 32 and info.workgroups == 8 * 32
     # fp32 causal B2 H8 N2048 (128-row tiles, two workgroups per CU): query
     # tiles paired, each tile in 4 ranges of its own length: 128 pairs x 4
     p = F.make_params(2, 8, 2048, 2048, 64, dtype=F.DTYPE_F32, causal=True)
