@@ -286,8 +286,10 @@ void no_key_split(const ofh_attention_params* p, Resolved& r) {
 // bias D64 non-causal H16 N1000 24 / 19, N1500 38 / 40, N2048 47 / 55). The
 // fewer the rows in all, the less a split has to merge (H32 M168 N2929 D128 32 /
 // 45, H2 N2500 29 / 32), hence the last factor. Few rows (one 128-row tile) leave groups without their gain (H64
-// M64 N1000 16 / 18), and grids of less than 32 128-row tiles keep the split,
-// on whose workspace and launch description their callers may rely.
+// M64 N1000 16 / 18). Grids of fewer than 32 128-row tiles keep the split over
+// workgroups; that is no line of time (D128 causal H9 N362 15.8 / 10.8, D64 H12 N186
+// 10.8 / 6.7): the tests of that split are written for such calls. A call that
+// sets max_key_splits, to whatever number, keeps the split's plans.
 void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
     if (p->dtype == OFH_DTYPE_F32 || p->max_key_splits != 0 || r.key_splits <= 1 || r.decode || r.tile_list ||
         r.kdim > 128 || p->query_tokens <= 128)
@@ -354,10 +356,14 @@ void choose_key_groups(const ofh_attention_params* p, Resolved& r) {
 // whole one (D64 H17 N1069, 578 blocks: 66 / 75), causal blocks in one round
 // wait for the longest (D128 H5 N826, 130 blocks: 37 / 38), and with fewer than
 // eight key tiles wavefronts stand idle (D128 H128 N183 37 / 41; causal rows far
-// past the last key see all of few keys: D128 H17 M3043 N281 112 / 124). Causal
-// pairs with a key split over more than 1024 keys keep that plan, on whose
-// workspace and launch description their callers may rely. So do more than three
-// rounds of fewer than 256 rows per head (D64 H128 M221 N1094 102 / 101).
+// past the last key see all of few keys: D128 H17 M3043 N281 112 / 124). Two
+// exclusions are no lines of time. Causal pairs with a key split over more than
+// 1024 keys keep that plan, which the planner's tests expect (D64 H18 N1430 84.0 /
+// 62.1, D128 H16 N1574 160 / 127, D64 B2 H8 N2048 103.6 / 96.5). More than three
+// rounds of fewer than 256 rows per head were left out for one call without a
+// gain (D64 H128 M221 N1094 102 / 101, causal 33.5 / 33.4) where others have one
+// (causal H200 M150 N1000 70.5 / 27.1, H128 M225 N500 69.0 / 53.3). A call that sets
+// max_key_splits, to whatever number, keeps the split's plans.
 void choose_f32_waves(const ofh_attention_params* p, Resolved& r) {
     if (p->dtype != OFH_DTYPE_F32 || p->max_key_splits != 0 || r.decode || r.general_mod || r.tile_list ||
         r.block_m == ofh::kRowsF32Narrow || (r.kdim != 64 && r.kdim != 128))

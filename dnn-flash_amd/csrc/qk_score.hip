@@ -37,7 +37,8 @@ __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 // product and sum are rounded separately, and the LDS: per k a thread reads 2 PT
 // floats for PT^2 multiply-adds. Measured, fp32 32 tiles 1024^2 x 128: 343 us
 // with 4 scores of one column per thread (a read per multiply-add, 64-bit index
-// arithmetic per load), 192 us with PT = 4 (45 TFLOP/s of useful work).
+// arithmetic per load), 195 us with PT = 4 (44 TFLOP/s of useful work; the ALU's rate,
+// one instruction per lane and multiply or add, allows 78).
 template <typename T, int PT>
 __global__ __launch_bounds__(256) void qk_score_kernel(QkScoreArgs a) {
     // Products, sums, scale and bias are each rounded: no contraction to FMA.

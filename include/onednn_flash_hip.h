@@ -118,7 +118,10 @@ typedef struct ofh_attention_params {
      * CPU loop has no workgroups to fill): a call whose query tiles give fewer
      * workgroups than the GPU holds runs each query tile's keys as several
      * workgroups and merges their partial rows. 0: the library chooses
-     * (ofh_launch_info.key_splits); 1: never split; n > 1: at most n splits. */
+     * (ofh_launch_info.key_splits); 1: never split; n > 1: at most n splits.
+     * Any n > 0, also one that restricts nothing, keeps the kernels of this
+     * split: the kernels that run mid-size calls in one workgroup per query
+     * tile instead are chosen with 0 only. */
     int32_t max_key_splits;
 } ofh_attention_params;
 
