@@ -24,7 +24,7 @@ def _need_gpu():
 
 
 @pytest.mark.parametrize("args,tol", [
-    (["--dtype", "f32"], 1e-5),                                            # reference defaults: D=32, rowwise kernel
+    (["--dtype", "f32"], 1e-5),                                            # reference defaults: D=32, 16-row fp32 blocks
     (["--dtype", "bf16", "--seq", "512", "--heads", "4", "--head-dim", "128"], 3e-2),
     (["--dtype", "f16", "--seq", "300", "--heads", "2", "--head-dim", "64", "--no-causal"], 5e-3),
 ])
