@@ -213,7 +213,7 @@ constexpr int kDecodeThreads = 512;
 // against 92.0 on the matrix cores (where the error against 64 bits is larger,
 // probabilities being rounded to bf16), 96.9 against 92.4 at four and 136
 // against 93 at eight. fp32 B16 H16 N4096 D64 stays at the memory's rate up to
-// eight (113 us; 90 at one row, against 300 on the matrix cores).
+// eight (111 us; 90 at one row, against 300 on the matrix cores).
 // 16-bit heads wider than 128 keep the matrix-core kernels (not measured here).
 inline int decode_max_rows(int dtype, int D, int Dv) {
     return dtype == DT_F32 ? 8 : D <= 128 && Dv <= 128 ? 2 : 0;
