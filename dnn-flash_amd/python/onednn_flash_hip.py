@@ -283,10 +283,8 @@ def dtype_code(t) -> int:
 
 
 def _raw_stream(torch, device) -> int:
-    """The current stream's handle on a GPU device; another device is refused here,
-    as torch.cuda.current_stream does (the score tile has no other check of it)."""
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
+    """The current stream's handle on a GPU device (the caller has checked that it
+    is one: another device's lookup would be the current GPU's)."""
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
@@ -440,6 +438,8 @@ def qk_score_tile(q, k, *, scale: float | None = None, bias=None, softcap: float
     N = k.shape[1]
     if k.shape[0] != T or k.shape[2] != D or k.dtype != q.dtype:
         raise ValueError("k must be [T, N, D] with the dtype of q")
+    if q.device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {q.device}")
     if out is None:
         out = torch.empty((T, M, N), device=q.device, dtype=torch.float32)
     p = QkScoreParams()
